@@ -76,6 +76,20 @@ def test_rmsnorm_backward_matches_oracle(ops, dtype, M, K):
     assert torch.equal(dx, dx2) and torch.equal(dw, dw2), "backward is not bitwise reproducible"
 
 
+@pytest.mark.parametrize("M,K", [(1, 8), (5, 40), (130, 1000), (2044, 24), (2048, 4096), (9000, 1800)])
+def test_rmsnorm_backward_dw_over_workgroup_counts(ops, M, K):
+    """dw where the row-group sum can go wrong: 1, 2, 33, 511 and 512 workgroup rows, and K off the 32-column blocks.
+    The bound is fp32's for a sum of M products: each term carries at most 2^-22, and every partial sum 2^-24."""
+    g = torch.Generator().manual_seed(M * K)
+    x, dy = torch.randn(M, K, generator=g), torch.randn(M, K, generator=g)
+    w = torch.randn(K, generator=g)
+    _, r = ops.rmsnorm(x.cuda(), w.cuda(), 1e-6)
+    _, dw = ops.rmsnorm_bwd(dy.cuda(), x.cuda(), w.cuda(), r)
+    terms = dy.double() * x.double() * r.cpu().double()[:, None]
+    bound = terms.abs().sum(0) * (2.0 ** -22 + M * 2.0 ** -24)
+    assert ((dw.cpu().double() - terms.sum(0)).abs() <= bound).all()
+
+
 def test_rmsnorm_module_autograd_under_autocast():
     from transformer_amd import RMSNorm
     g = torch.Generator().manual_seed(9)
