@@ -437,6 +437,28 @@ typedef struct {
 } mla_norm_linear_args;
 int mla_norm_linear(const mla_norm_linear_args* a, void* stream);
 
+/* --------------------------------------------------------- weight_grad --
+ * dw[n][k] = sum_m dy[m][n] x[m][k]: the gradient of a linear layer's weight [N, K] from its output
+ * gradient dy [M, N] and its input x [M, K] (bf16 token rows with row strides), fp32 sums, fp32 or
+ * bf16 dw [N, K] (row stride dw_stride).  M < 2^24; N, K and the strides of dy and x multiples of 8,
+ * their pointers 16-byte aligned; (M + 256) rows of either operand below 2 GiB.  The workspace holds
+ * the fp32 partials of the token segments (0 bytes when one segment fills the GPU).
+ *
+ * Replaces: autograd of the projections at transformer.py:208-213, :263, :300 and of the loss's
+ *           logits at :96-98 with respect to their weights.
+ */
+typedef struct {
+  const void* dy;
+  const void* x;
+  void* dw;
+  void* workspace;
+  size_t workspace_bytes;
+  int64_t M, N, K, dy_stride, x_stride, dw_stride;
+  int32_t dw_dtype;
+} mla_weight_grad_args;
+size_t mla_weight_grad_workspace_bytes(const mla_weight_grad_args* a);
+int mla_weight_grad(const mla_weight_grad_args* a, void* stream);
+
 /* ---------------------------------------------------- chunked linear CE --
  * One vocabulary chunk of the exact softmax cross-entropy over tied output weights, given
  * that chunk's logits [N, Vc] (row stride ld) = x . W[v0 : v0 + Vc]^T of `dtype`
@@ -473,7 +495,8 @@ int mla_ce_chunk(const mla_ce_chunk_args* a, void* stream);
  * mla_abi_version: MLA_ABI_VERSION of the built library.
  * mla_args_size: sizeof() of the argument structs, for binding checks
  *   (0 rope, 1 prefill_fwd, 2 prefill_bwd, 3 decode, 4 rmsnorm, 5 rmsnorm_bwd, 6 decode_out,
- *    7 rope_append, 8 absorb_q, 9 ce_chunk, 10 linear_rows, 11 prefill_cached, 12 norm_linear).
+ *    7 rope_append, 8 absorb_q, 9 ce_chunk, 10 linear_rows, 11 prefill_cached, 12 norm_linear,
+ *    13 weight_grad).
  */
 const char* mla_last_error(void);
 int mla_abi_version(void);

@@ -1,0 +1,119 @@
+"""mla_weight_grad (dW = dY^T X) and the training branch's linear layers built on it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("out_fp32", [True, False])
+@pytest.mark.parametrize("M,N,K,pad", [
+    (1, 8, 8, 0),            # one token, one 16-byte chunk
+    (31, 264, 136, 0),       # a ragged only stage, past one tile both ways
+    (32, 256, 128, 8),       # one full stage, strided rows
+    (33, 256, 256, 0),       # a one-token tail
+    (97, 1000, 392, 24),     # four stages (the ring's depth) with a tail
+    (160, 256, 256, 0),      # five stages: one through the steady loop
+    (1000, 2624, 2048, 0),   # one segment of wide or narrow tiles
+    (4100, 384, 1792, 16),   # many segments, the last one ragged
+    (12288, 896, 384, 0),    # the segments' partials read eight at a time, and a remainder
+])
+def test_weight_grad_matches_fp64(M, N, K, pad, out_fp32):
+    from transformer_amd import kernels
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    by = torch.randn(M, N + 2 * pad, generator=g, device="cuda").bfloat16()
+    bx = torch.randn(M, K + 2 * pad, generator=g, device="cuda").bfloat16()
+    dy, x = by[:, pad:pad + N], bx[:, pad:pad + K]
+    dw = kernels.weight_grad(dy, x, out_fp32)
+    ref = dy.double().t().contiguous() @ x.double().contiguous()
+    # fp32 sums of M exact products: at most M 2^-24 of the sum of magnitudes; then one rounding to bf16
+    mag = dy.double().abs().t().contiguous() @ x.double().abs().contiguous()
+    bound = mag * (M + 8) * 2.0 ** -24
+    if not out_fp32:
+        bound = bound + (ref.abs() + bound) * 2.0 ** -8
+    assert dw.dtype == (torch.float32 if out_fp32 else torch.bfloat16) and dw.shape == (N, K)
+    assert ((dw.double() - ref).abs() <= bound).all()
+    assert torch.equal(dw, kernels.weight_grad(dy, x, out_fp32)), "not bitwise reproducible"
+
+
+def test_weight_grad_keeps_infinities_to_their_rows_and_the_padding_out():
+    # 37 tokens: the stage's rows past the end and the columns past N and K hold NaN in memory
+    from transformer_amd import kernels
+    by = torch.full((64, 64), float("nan"), device="cuda").bfloat16()
+    bx = torch.full((64, 64), float("nan"), device="cuda").bfloat16()
+    by[:37, :24], bx[:37, :40] = 1, 1
+    by[36, 3], bx[5, 7] = float("inf"), float("-inf")
+    dw = kernels.weight_grad(by[:37, :24], bx[:37, :40], True).cpu()
+    ref = torch.full((24, 40), 37.0)
+    ref[3, :], ref[:, 7] = float("inf"), float("-inf")
+    ref[3, 7] = float("nan")
+    assert torch.equal(torch.nan_to_num(dw, nan=123.0), torch.nan_to_num(ref, nan=123.0))
+
+
+def test_weight_grad_rejects_what_it_does_not_take():
+    from transformer_amd import kernels
+    z = lambda *s, dt=torch.bfloat16: torch.zeros(*s, dtype=dt, device="cuda")
+    for dy, x, err in ((z(4, 12), z(4, 8), ValueError), (z(4, 8), z(4, 20), ValueError), (z(4, 8), z(5, 8), ValueError),
+                       (z(0, 8), z(0, 8), ValueError), (z(4, 8, dt=torch.float32), z(4, 8), TypeError)):
+        with pytest.raises(err):
+            kernels.weight_grad(dy, x)
+
+
+@pytest.mark.parametrize("amp", [True, False])
+@pytest.mark.parametrize("frozen", [(), ("q_up", "kv_down"), ("q_down", "qk_rope", "kv_down")])
+def test_module_gradients_equal_torch_layers(monkeypatch, amp, frozen):
+    """The training branch's linear layers against the same module on torch's own (what a hook on each makes it take),
+    for fp32 weights under autocast and bf16 weights, with frozen weights: each gradient within bf16's rounding."""
+    from transformer_amd import MLA, ModelArgs, training
+    g = torch.Generator(device="cuda").manual_seed(3)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs(max_seq_len=256))
+    for p in m.parameters():
+        p.data.copy_(torch.randn(p.shape, generator=g, device="cuda") * 0.02)
+    m = m if amp else m.to(torch.bfloat16)
+    for n in frozen:
+        m._modules[n].weight.requires_grad_(False)
+    x0 = torch.randn(2, 150, m.d_model, generator=g, device="cuda").to(torch.bfloat16)
+    dy = torch.randn(2, 150, m.d_model, generator=g, device="cuda").to(torch.bfloat16)
+
+    def run():
+        m.zero_grad(set_to_none=True)
+        x = x0.clone().requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            y, _ = m(x)
+        y.backward(dy)
+        return [y.detach(), x.grad] + [p.grad for p in m.parameters()]
+
+    calls = []
+    real = training.linear
+    monkeypatch.setattr(training, "linear", lambda *a, **k: calls.append(1) or real(*a, **k))
+    ours = run()
+    assert calls
+    monkeypatch.setattr(training, "plain_call", lambda *t: False)
+    n = len(calls)
+    theirs = run()
+    assert len(calls) == n
+    for a, b in zip(ours, theirs):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert a.dtype == b.dtype and a.shape == b.shape
+            assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
+
+
+def test_linear_double_backward_and_hooked_layers():
+    """create_graph through a layer alone (what torch's layer allows), and a hooked layer keeps its call."""
+    from transformer_amd import training
+    lin = torch.nn.Linear(64, 128, bias=False, device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(5, 64, device="cuda").bfloat16().requires_grad_(True)
+    assert training.takes(lin, x)
+
+    def penalty(f):
+        gx, gw = torch.autograd.grad(f(x).square().sum(), (x, lin.weight), create_graph=True)
+        return torch.autograd.grad(gx.float().square().sum() + gw.float().square().sum(), (x, lin.weight))
+
+    for a, b in zip(penalty(lambda t: training.linear(t, lin.weight)), penalty(lin)):
+        assert (a.double() - b.double()).norm() <= 2e-2 * b.double().norm()
+    h = lin.register_forward_hook(lambda *a: None)
+    assert not training.takes(lin, x)
+    h.remove()
+    with torch.no_grad():
+        assert not training.takes(lin, x)

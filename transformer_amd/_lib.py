@@ -166,9 +166,17 @@ class RmsNormBwdArgs(ctypes.Structure):
     ]
 
 
+class WeightGradArgs(ctypes.Structure):
+    _fields_ = [
+        ("dy", c_void_p), ("x", c_void_p), ("dw", c_void_p), ("workspace", c_void_p), ("workspace_bytes", c_size_t),
+        ("M", c_int64), ("N", c_int64), ("K", c_int64), ("dy_stride", c_int64), ("x_stride", c_int64),
+        ("dw_stride", c_int64), ("dw_dtype", c_int32),
+    ]
+
+
 ARGS_STRUCTS = {0: RopeArgs, 1: PrefillFwdArgs, 2: PrefillBwdArgs, 3: DecodeArgs, 4: RmsNormArgs,
                 5: RmsNormBwdArgs, 6: DecodeOutArgs, 7: RopeAppendArgs, 8: AbsorbQArgs, 9: CeChunkArgs,
-                10: LinearRowsArgs, 11: PrefillCachedArgs, 12: NormLinearArgs}
+                10: LinearRowsArgs, 11: PrefillCachedArgs, 12: NormLinearArgs, 13: WeightGradArgs}
 
 # exported symbol -> (restype, argtypes)
 SIGNATURES = {
@@ -184,6 +192,8 @@ SIGNATURES = {
     "mla_decode_static": (c_int, [POINTER(DecodeArgs), c_void_p]),
     "mla_absorb_q": (c_int, [POINTER(AbsorbQArgs), c_void_p]),
     "mla_norm_linear": (c_int, [POINTER(NormLinearArgs), c_void_p]),
+    "mla_weight_grad_workspace_bytes": (c_size_t, [POINTER(WeightGradArgs)]),
+    "mla_weight_grad": (c_int, [POINTER(WeightGradArgs), c_void_p]),
     "mla_prefill_cached_workspace_bytes": (c_size_t, [POINTER(PrefillCachedArgs)]),
     "mla_prefill_cached": (c_int, [POINTER(PrefillCachedArgs), c_void_p]),
     "mla_decode_out_workspace_bytes": (c_size_t, [POINTER(DecodeOutArgs)]),

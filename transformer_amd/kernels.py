@@ -915,6 +915,39 @@ def _rms_backward(ctx, dy, dinv):
 rmsnorm.register_autograd(_rms_backward, setup_context=_rms_setup)
 
 
+# ----------------------------------------------------------------- weight gradient
+
+def weight_grad_fits(M: int, N: int, K: int, dy_stride: int, x_stride: int) -> bool:
+    """Whether a [M, N]^T x [M, K] product is within weight_grad's limits (see mla_mi355x.h)."""
+    return 0 < M < 1 << 24 and 0 < N < 1 << 20 and 0 < K < 1 << 20 and N % 8 == 0 and K % 8 == 0 \
+        and (M + 256) * max(dy_stride, x_stride) * 2 < 1 << 31
+
+
+def weight_grad(dy: Tensor, x: Tensor, out_fp32: bool = False) -> Tensor:
+    """``dy^T x`` for bf16 ``dy [M, N]`` and ``x [M, K]`` (unit inner stride): the gradient ``[N, K]`` of a linear
+    layer's weight (the autograd of transformer.py:208-213, :263, :300), fp32 sums, rounded once to bf16 or, with
+    ``out_fp32``, not at all.  Not a registered operator: it is called inside backward passes only."""
+    op = "mla_mi355x::weight_grad"
+    _require_gpu(op, dy, x)
+    _bf16(op, dy=dy, x=x)
+    if dy.dim() != 2 or x.dim() != 2 or dy.size(0) != x.size(0):
+        raise ValueError(f"{op}: expected dy [M, N] and x [M, K]; got {tuple(dy.shape)}, {tuple(x.shape)}")
+    dy, x = _aligned4(dy, 8), _aligned4(x, 8)
+    (M, N), K = dy.shape, x.size(1)
+    sy, sx = (dy.stride(0), x.stride(0)) if M > 1 else (N, K)
+    if not weight_grad_fits(M, N, K, sy, sx):
+        raise ValueError(f"{op}: M = {M}, N = {N}, K = {K} with row strides {sy}, {sx} is outside the kernel's limits")
+    dw = torch.empty(N, K, dtype=torch.float32 if out_fp32 else torch.bfloat16, device=dy.device)
+    args = _lib.WeightGradArgs(dy=dy.data_ptr(), x=x.data_ptr(), dw=dw.data_ptr(), workspace=None, workspace_bytes=0,
+                               M=M, N=N, K=K, dy_stride=sy, x_stride=sx, dw_stride=K, dw_dtype=_dt_code(dw))
+    nbytes = int(_lib.entry("mla_weight_grad_workspace_bytes")(ctypes.byref(args)))
+    if nbytes:
+        ws = _alloc_workspace(nbytes, dy.device)
+        args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
+    _lib.check(_lib.entry("mla_weight_grad")(ctypes.byref(args), _stream(dw)), op)
+    return dw
+
+
 # ----------------------------------------------------------------- chunked linear cross-entropy
 
 def _ce_check(op: str, logits: Tensor, targets: Tensor, lse: Tensor) -> Tuple[int, int]:

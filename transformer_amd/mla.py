@@ -38,6 +38,7 @@ import torch.nn as nn
 
 from . import kernels  # noqa: F401  (registers the ops)
 from . import latent_cache
+from . import training
 from .decode_graph import DecodeGraph, autocast_bf16
 from .config import mla_dims
 
@@ -100,23 +101,11 @@ def _linear_split_cols(x, W):
     return y.view(*x.shape[:-1], N)
 
 
-class _SplitColsLinear(torch.autograd.Function):
-    """``x @ W^T`` with the forward as _linear_split_cols and the backward as single products
-    (the split does not pay there: dx 214 against 243 us, dW 336 against 397 us at the benchmark
-    down-projections)."""
-
-    @staticmethod
-    def forward(ctx, x, W):
-        ctx.save_for_backward(x, W)
+def _down_product(x, W):
+    """``x @ W^T`` of the down-projections, as two products where that pays."""
+    if _split_pays(x.numel() // x.size(-1), W.size(0)):
         return _linear_split_cols(x, W)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, W = ctx.saved_tensors
-        dy2 = dy.reshape(-1, dy.size(-1))
-        dx = (dy2 @ W).view(x.shape) if ctx.needs_input_grad[0] else None
-        dW = dy2.t() @ x.reshape(-1, x.size(-1)) if ctx.needs_input_grad[1] else None
-        return dx, dW
+    return torch.nn.functional.linear(x, W)
 
 
 class RotaryEmbedding(nn.Module):
@@ -321,23 +310,33 @@ class MLA(nn.Module):
         ws = (self.q_down.weight, self.qk_rope.weight, self.kv_down.weight)
         sizes = [w.size(0) for w in ws]
         split = _split_pays(x.numel() // x.size(-1), sum(sizes)) and not torch.compiler.is_compiling()
+        amp = torch.is_autocast_enabled("cuda")
         if torch.is_grad_enabled() and any(w.requires_grad for w in ws):
-            W = torch.cat(ws, 0)
-            if split:  # autocast's casts, made explicit for the autograd Function
-                dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else W.dtype
-                return _SplitColsLinear.apply(x.to(dt), W.to(dt)).split(sizes, dim=-1)
-        else:
-            dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else ws[0].dtype
-            key = tuple((w.data_ptr(), w._version) for w in ws) + (dt,)
-            if getattr(self, "_down_key", None) != key:
-                self._down_w = torch.cat([w.detach() for w in ws], 0).to(dt)
-                self._down_key = key
-            W = self._down_w
-        if not split or W.requires_grad:
+            # autocast's casts, made explicit for the autograd Function.  The split does not pay in the backward (dx
+            # 214 against 243 us at the benchmark down-projections), whose products are single ones
+            dt = torch.get_autocast_dtype("cuda") if amp else \
+                torch.promote_types(torch.promote_types(ws[0].dtype, ws[1].dtype), ws[2].dtype)
+            if (split or (dt == torch.bfloat16 and (amp or x.dtype == dt))) and training.plain_call(x, *ws):
+                return training.linear(x.to(dt), *ws, product=_down_product).split(sizes, dim=-1)
+            return torch.nn.functional.linear(x, torch.cat(ws, 0)).split(sizes, dim=-1)
+        dt = torch.get_autocast_dtype("cuda") if amp else ws[0].dtype
+        key = tuple((w.data_ptr(), w._version) for w in ws) + (dt,)
+        if getattr(self, "_down_key", None) != key:
+            self._down_w = torch.cat([w.detach() for w in ws], 0).to(dt)
+            self._down_key = key
+        W = self._down_w
+        if not split:
             return torch.nn.functional.linear(x, W).split(sizes, dim=-1)
         if torch.is_grad_enabled() and x.requires_grad:  # frozen weights, the input's gradient
-            return _SplitColsLinear.apply(x.to(W.dtype), W).split(sizes, dim=-1)
+            return training.linear(x.to(W.dtype), W, product=_down_product).split(sizes, dim=-1)
         return _linear_split_cols(x.to(W.dtype), W).split(sizes, dim=-1)
+
+    def _proj(self, name, x):
+        """``self.<name>(x)``, with the weight gradient on this package's kernel where that is all the layer does."""
+        m = self._modules[name]
+        if training.takes(m, x):
+            return training.linear(x.to(torch.bfloat16), m.weight)
+        return m(x)
 
     @staticmethod
     def _bf16(t):
@@ -384,7 +383,7 @@ class MLA(nn.Module):
             q_content = ops.linear_rows(q_low.reshape(B * T, -1), Wq).view(B, T, -1)  # :208
         else:
             q_low, qk_pos, kv_new = self._down_proj(x)  # :208-213, one GEMM (see _down_proj)
-            q_content = self.q_up(q_low)  # [B,T,H*dn]                   :208
+            q_content = self._proj("q_up", q_low)  # [B,T,H*dn]                   :208
         cdt = q_content.dtype
 
         q_nope = q_content.view(B, T, H, dn)
@@ -424,8 +423,8 @@ class MLA(nn.Module):
             k_rope = k_rope.transpose(1, 2)
         else:
             kv_latent, k_rope = kv_new, k_rope_new
-        k_nope = self.k_up(kv_latent).view(B, kv_len, H, dn)
-        v = self.v_up(kv_latent).view(B, kv_len, H, dv)
+        k_nope = self._proj("k_up", kv_latent).view(B, kv_len, H, dn)
+        v = self._proj("v_up", kv_latent).view(B, kv_len, H, dv)
         b = self._bf16
         if q_rope is None:
             o, _, _ = ops.prefill_fwd_rope(b(q_nope), qk4[:, :, :H], b(k_nope), b(k_rope), b(v), cos, sin, self.scale,
@@ -433,7 +432,7 @@ class MLA(nn.Module):
         else:
             o, _ = ops.prefill_fwd(b(q_nope), b(q_rope), b(k_nope), b(k_rope), b(v), self.scale, True, 0)
         out = o.reshape(B, T, H * dv).to(cdt)
-        return self.o_proj(out), None
+        return self._proj("o_proj", out), None
 
     def _forward_cached(self, x, q_nope, q_rope, k_rope_new, kv_new, kv_cache, pos_offset, cdt, appended=None,
                         rows=False):
