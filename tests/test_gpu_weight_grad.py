@@ -59,14 +59,15 @@ def test_weight_grad_rejects_what_it_does_not_take():
 
 
 @pytest.mark.parametrize("amp", [True, False])
-@pytest.mark.parametrize("frozen", [(), ("q_up", "kv_down"), ("q_down", "qk_rope", "kv_down")])
-def test_module_gradients_equal_torch_layers(monkeypatch, amp, frozen):
+@pytest.mark.parametrize("frozen", [(), ("q_up", "kv_down"), ("q_down", "qk_rope", "kv_down"), ("k_up",)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_module_gradients_equal_torch_layers(monkeypatch, amp, frozen, shared):
     """The training branch's linear layers against the same module on torch's own (what a hook on each makes it take),
     for fp32 weights under autocast and bf16 weights, with frozen weights: each gradient within bf16's rounding."""
     from transformer_amd import MLA, ModelArgs, training
     g = torch.Generator(device="cuda").manual_seed(3)
     with torch.device("cuda"):
-        m = MLA(ModelArgs(max_seq_len=256))
+        m = MLA(ModelArgs.mla_baseline(max_seq_len=256) if shared else ModelArgs(max_seq_len=256))
     for p in m.parameters():
         p.data.copy_(torch.randn(p.shape, generator=g, device="cuda") * 0.02)
     m = m if amp else m.to(torch.bfloat16)
@@ -97,6 +98,35 @@ def test_module_gradients_equal_torch_layers(monkeypatch, amp, frozen):
         if a is not None:
             assert a.dtype == b.dtype and a.shape == b.shape
             assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
+
+
+def _small(**over):
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(5)
+    with torch.device("cuda"):
+        return MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=128, **over)).to(
+            torch.bfloat16)
+
+
+def test_attention_function_under_saved_tensor_hooks_checkpoint_and_create_graph():
+    """What autograd offers around the training branch works as around the operators: saved-tensor hooks, activation
+    checkpointing, gradients through o_proj's own gradient, and the refusal to differentiate the attention twice."""
+    m = _small()
+    x = torch.randn(1, 70, 256, device="cuda").bfloat16().requires_grad_(True)
+    dy = torch.randn_like(x)
+    leaves = [x] + list(m.parameters())
+    want = torch.autograd.grad(m(x)[0], leaves, dy)
+    with torch.autograd.graph.save_on_cpu():
+        got = torch.autograd.grad(m(x)[0], leaves, dy)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+    y = torch.utils.checkpoint.checkpoint(lambda t: m(t)[0], x, use_reentrant=False)
+    assert all(torch.equal(a, b) for a, b in zip(want, torch.autograd.grad(y, leaves, dy)))
+    (g,) = torch.autograd.grad(m(x)[0], [m.o_proj.weight], dy, create_graph=True)
+    second = torch.autograd.grad(g.float().square().sum(), [x, m.v_up.weight])
+    assert all(torch.isfinite(t).all() and t.abs().max() > 0 for t in second)
+    (g,) = torch.autograd.grad(m(x)[0], [x], dy, create_graph=True)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(g.float().square().sum(), [x])
 
 
 def test_linear_double_backward_and_hooked_layers():

@@ -148,3 +148,48 @@ def test_backward_stored_ds_workspace_counts_the_visible_blocks():
             (B, H, Tq, Tk, q_offset, causal)
     full, small = sizes(16, 16, 16384, 16384, 0, True)  # 17.2 GB of dS blocks: over the cap, recompute path
     assert full == small
+
+
+def test_autograd_functions_stand_in_only_in_plain_eager_mode():
+    # the eager calls' autograd.Functions (and the training branch's) give way to the registered operators wherever
+    # something would see less: a trace, a mode, a transform, forward-mode, tensors that are not plain
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.overrides import TorchFunctionMode
+    from transformer_amd import kernels
+    fits = kernels.function_fits
+    assert fits(()) and fits((1, None)) and not fits((torch.zeros(2),)) and not fits((torch.zeros(2, device="meta"),))
+    with FakeTensorMode():
+        assert not fits(())
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert not fits(())
+    with torch.autograd.forward_ad.dual_level():
+        assert not fits(())
+    seen = []
+    torch.func.grad(lambda t: (seen.append(fits(())), t.sum())[1])(torch.zeros(3))
+    torch.jit.trace(lambda t: (seen.append(fits(())), t + 1)[1], torch.zeros(3), check_trace=False)
+    assert seen and not any(seen)
+    assert torch.compile(lambda t: t + (-1 if fits(()) else 1), backend="eager", fullgraph=True)(torch.zeros(1)).item() == 1
+
+
+def test_training_layers_take_only_plain_linears():
+    from transformer_amd import training
+    lin = torch.nn.Linear(8, 8, bias=False)
+    assert training.plain_linear(lin)
+    assert not training.plain_linear(torch.nn.Linear(8, 8)) and not training.plain_linear(torch.nn.Identity())
+    sub = type("Sub", (torch.nn.Linear,), {})(8, 8, bias=False)
+    assert not training.plain_linear(sub)
+    for hook in (lin.register_forward_pre_hook, lin.register_forward_hook, lin.register_full_backward_hook):
+        h = hook(lambda *a: None)
+        assert not training.plain_linear(lin)
+        h.remove()
+    h = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert not training.plain_linear(lin)
+    h.remove()
+    assert training.plain_linear(lin)
+    torch.nn.utils.parametrizations.weight_norm(lin)
+    assert not training.plain_linear(lin)

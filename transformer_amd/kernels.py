@@ -12,6 +12,7 @@ There is no CPU path: a CPU tensor, or a missing library, raises.
 from __future__ import annotations
 
 import ctypes
+import inspect
 from typing import Optional, Tuple
 
 import torch
@@ -33,6 +34,8 @@ BWD_STORED_DS = True
 
 # the op bodies by name, as registered: ``eager`` below calls them without the dispatcher
 _BODIES = {}
+# the autograd formulas by name (setup_context, backward), as registered
+_FORMULAS = {}
 
 
 def _op(name: str, mutates_args=()):
@@ -41,6 +44,11 @@ def _op(name: str, mutates_args=()):
         _BODIES[name] = fn
         return torch.library.custom_op(f"mla_mi355x::{name}", mutates_args=mutates_args)(fn)
     return register
+
+
+def _register_autograd(op, name: str, setup, backward) -> None:
+    op.register_autograd(backward, setup_context=setup)
+    _FORMULAS[name] = (setup, backward)
 
 
 def _require_gpu(op: str, *tensors: Tensor) -> None:
@@ -133,10 +141,10 @@ def _rope_setup(ctx, inputs, output):
 def _rope_backward(ctx, grad):
     cos, sin = ctx.saved_tensors
     # R is orthogonal: the gradient is the rotation by the opposite angle
-    return torch.ops.mla_mi355x.rope(grad, cos, sin, ctx.pos_offset, not ctx.inverse), None, None, None, None
+    return eager.rope(grad, cos, sin, ctx.pos_offset, not ctx.inverse), None, None, None, None
 
 
-rope.register_autograd(_rope_backward, setup_context=_rope_setup)
+_register_autograd(rope, "rope", _rope_setup, _rope_backward)
 
 
 @_op("rope_", mutates_args=("x",))
@@ -340,6 +348,13 @@ def prefill_bwd(dout: Tensor, q_nope: Tensor, q_rope: Tensor, k_nope: Tensor, k_
     over query heads.  With ``cos``/``sin`` (the backward of :func:`prefill_fwd_rope`),
     ``q_rope`` is the rotated slice and dq_rope is returned for the unrotated one, rotated
     back at positions ``q_pos_offset + t`` in the dQ kernel before its rounding."""
+    return _prefill_bwd_impl(dout, q_nope, q_rope, k_nope, k_rope, v, o, lse, scale, causal, q_offset, cos, sin,
+                             q_pos_offset)
+
+
+def _prefill_bwd_impl(dout, q_nope, q_rope, k_nope, k_rope, v, o, lse, scale, causal, q_offset, cos=None, sin=None,
+                      q_pos_offset=0, out=None):
+    """``out``: the five gradients' tensors (16-byte aligned rows of any strides), by default new ones."""
     op = "mla_mi355x::prefill_bwd"
     B, Tq, Tk, H, Hr, dn, dv = _prefill_check(op, q_nope, q_rope, k_nope, k_rope, v)
     _require_gpu(op, dout, o, lse)
@@ -350,11 +365,10 @@ def prefill_bwd(dout: Tensor, q_nope: Tensor, q_rope: Tensor, k_nope: Tensor, k_
     dout, q_nope, q_rope, k_nope, k_rope, v, o = (_aligned4(t, 8) for t in (dout, q_nope, q_rope, k_nope, k_rope, v, o))
     lse = lse.contiguous()
     dev = q_nope.device
-    dq_nope = torch.empty(B, Tq, H, dn, dtype=torch.bfloat16, device=dev)
-    dq_rope = torch.empty(B, Tq, H, ROPE_DIM, dtype=torch.bfloat16, device=dev)
-    dk_nope = torch.empty(B, Tk, H, dn, dtype=torch.bfloat16, device=dev)
-    dk_rope = torch.empty(B, Tk, Hr, ROPE_DIM, dtype=torch.bfloat16, device=dev)
-    dvv = torch.empty(B, Tk, H, dv, dtype=torch.bfloat16, device=dev)
+    if out is None:
+        out = [torch.empty(*shape, dtype=torch.bfloat16, device=dev) for shape in (
+            (B, Tq, H, dn), (B, Tq, H, ROPE_DIM), (B, Tk, H, dn), (B, Tk, Hr, ROPE_DIM), (B, Tk, H, dv))]
+    dq_nope, dq_rope, dk_nope, dk_rope, dvv = out
     if dq_nope.numel() == 0 and dk_nope.numel() == 0:
         return dq_nope, dq_rope, dk_nope, dk_rope, dvv
     args = PrefillBwdArgs(
@@ -419,12 +433,11 @@ def _prefill_setup(ctx, inputs, output):
 
 def _prefill_backward(ctx, do, dlse):
     q_nope, q_rope, k_nope, k_rope, v, o, lse = ctx.saved_tensors
-    grads = torch.ops.mla_mi355x.prefill_bwd(do, q_nope, q_rope, k_nope, k_rope, v, o, lse,
-                                             ctx.scale, ctx.causal, ctx.q_offset)
+    grads = eager.prefill_bwd(do, q_nope, q_rope, k_nope, k_rope, v, o, lse, ctx.scale, ctx.causal, ctx.q_offset)
     return (*grads, None, None, None)
 
 
-prefill_fwd.register_autograd(_prefill_backward, setup_context=_prefill_setup)
+_register_autograd(prefill_fwd, "prefill_fwd", _prefill_setup, _prefill_backward)
 
 
 def _prefill_rope_setup(ctx, inputs, output):
@@ -440,12 +453,12 @@ def _prefill_rope_backward(ctx, do, dlse, dqrot):
     if not ctx.saved_rotated:
         raise RuntimeError("prefill_fwd_rope: the backward needs save_rotated=True in the forward")
     q_nope, q_rot, k_nope, k_rope, v, o, lse, cos, sin = ctx.saved_tensors
-    grads = torch.ops.mla_mi355x.prefill_bwd(do, q_nope, q_rot, k_nope, k_rope, v, o, lse, ctx.scale, ctx.causal,
-                                             ctx.q_offset, cos, sin, ctx.q_pos_offset)
+    grads = eager.prefill_bwd(do, q_nope, q_rot, k_nope, k_rope, v, o, lse, ctx.scale, ctx.causal, ctx.q_offset, cos,
+                              sin, ctx.q_pos_offset)
     return (*grads, None, None, None, None, None, None, None)
 
 
-prefill_fwd_rope.register_autograd(_prefill_rope_backward, setup_context=_prefill_rope_setup)
+_register_autograd(prefill_fwd_rope, "prefill_fwd_rope", _prefill_rope_setup, _prefill_rope_backward)
 
 
 # ----------------------------------------------------------------- decode
@@ -908,11 +921,11 @@ def _rms_setup(ctx, inputs, output):
 
 def _rms_backward(ctx, dy, dinv):
     x, weight, inv = ctx.saved_tensors
-    dx, dw = torch.ops.mla_mi355x.rmsnorm_bwd(dy, x, weight, inv)
+    dx, dw = eager.rmsnorm_bwd(dy, x, weight, inv)
     return dx, dw.to(weight.dtype), None, None
 
 
-rmsnorm.register_autograd(_rms_backward, setup_context=_rms_setup)
+_register_autograd(rmsnorm, "rmsnorm", _rms_setup, _rms_backward)
 
 
 # ----------------------------------------------------------------- weight gradient
@@ -1010,6 +1023,21 @@ def _(logits, targets, lse, g_vec, g_scale, v0):
 
 # ----------------------------------------------------------------- eager calls
 
+def _not_plain(args) -> bool:
+    """Tracing (torch.compile), a dispatch mode, a functorch transform, tensor subclasses, or tensors off the GPU."""
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 \
+            or torch._C._functorch.peek_interpreter_stack() is not None:
+        return True
+    for a in args:
+        if isinstance(a, Tensor) and ((type(a) is not Tensor and type(a) is not torch.nn.Parameter) or not a.is_cuda):
+            return True
+    return False
+
+
+def _needs_grad(args) -> bool:
+    return torch.is_grad_enabled() and any(isinstance(a, Tensor) and a.requires_grad for a in args)
+
+
 def dispatcher_needed(args) -> bool:
     """Whether a call with ``args`` must go through the registered operator: under tracing
     (torch.compile), a dispatch mode (fake tensors, functionalization), a functorch transform,
@@ -1017,25 +1045,51 @@ def dispatcher_needed(args) -> bool:
     that needs a gradient while grad mode is on (the autograd formulas live on the
     operators).  Otherwise the operator adds only dispatch time (about 15 us of Python per
     call) around the same body."""
-    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 \
-            or torch._C._functorch.peek_interpreter_stack() is not None:
-        return True
-    grad = torch.is_grad_enabled()
-    for a in args:
-        if isinstance(a, Tensor):
-            if (type(a) is not Tensor and type(a) is not torch.nn.Parameter) or not a.is_cuda:
-                return True
-            if grad and a.requires_grad:
-                return True
-    return False
+    return _not_plain(args) or _needs_grad(args)
+
+
+def function_fits(args) -> bool:
+    """Whether an autograd.Function may stand in for a registered operator whose gradient is needed: nothing else in
+    :func:`dispatcher_needed` holds, and no forward-mode level, jit trace or torch-function mode would see less."""
+    return torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_function_stack() == 0 \
+        and torch._C._get_tracing_state() is None and not _not_plain(args)
+
+
+def below_autograd():
+    """The guard under which torch runs an operator's body, for the same body inside an autograd.Function."""
+    return torch._C._AutoDispatchBelowAutograd()
+
+
+def _function(name: str):
+    """The autograd.Function of the operator ``name``: its body and registered formulas, which see the same inputs,
+    outputs and saved tensors as under the operator.  The operator's own autograd costs 60 to 80 us of host time a
+    call, and its backward makes zeros for the outputs that have no gradient."""
+    setup, backward = _FORMULAS[name]
+    body = _BODIES[name]
+
+    def forward(*args):
+        with below_autograd():
+            return body(*args)
+
+    def setup_context(ctx, inputs, output):
+        ctx.set_materialize_grads(False)
+        setup(ctx, inputs, output)
+
+    return type("_" + name, (torch.autograd.Function,), {
+        "forward": staticmethod(forward), "setup_context": staticmethod(setup_context),
+        "backward": staticmethod(backward)})
 
 
 def _eager_call(name: str):
     body = _BODIES[name]
     op = getattr(torch.ops.mla_mi355x, name)
+    fn = _function(name) if name in _FORMULAS else None
+    n_args = len(inspect.signature(body).parameters)
 
     def call(*args, **kwargs):
         if dispatcher_needed(args) or (kwargs and dispatcher_needed(kwargs.values())):
+            if fn is not None and not kwargs and len(args) == n_args and function_fits(args):
+                return fn.apply(*args)
             return op(*args, **kwargs)
         return body(*args, **kwargs)
 
@@ -1046,7 +1100,8 @@ def _eager_call(name: str):
 
 class _EagerOps:
     """``torch.ops.mla_mi355x`` for eager callers: each attribute runs the operator's own body
-    directly when ``dispatcher_needed`` is false, else the registered operator."""
+    directly when ``dispatcher_needed`` is false, its autograd formula as a plain autograd.Function
+    when a gradient is all that is needed, else the registered operator."""
 
     def __init__(self):
         for name in _BODIES:

@@ -301,15 +301,19 @@ class MLA(nn.Module):
         return self.o_proj.weight.dtype == torch.bfloat16
 
     def _down_proj(self, x):
+        """The column views of :meth:`_down_all`: ``q_down(x)``, ``qk_rope(x)`` and ``kv_down(x)``."""
+        return self._down_all(x).split([self.q_down.weight.size(0), self.qk_rope.weight.size(0),
+                                        self.kv_down.weight.size(0)], dim=-1)
+
+    def _down_all(self, x):
         """``q_down(x)``, ``qk_rope(x)`` and ``kv_down(x)`` (transformer.py:208-213) as one GEMM
         over the concatenated weights ``[q_lora + (H + Hr) 64 + d_latent, d_model]``: x is read
-        once instead of three times.  The outputs are column views of the one result.  With
+        once instead of three times.  With
         autograd off the concatenation (in the autocast dtype) is kept while the three
         weights are unchanged.  For many rows and N past a multiple of 256 (2624 at the
         ModelArgs.mla_baseline dims) the forward product runs as two (_linear_split_cols)."""
         ws = (self.q_down.weight, self.qk_rope.weight, self.kv_down.weight)
-        sizes = [w.size(0) for w in ws]
-        split = _split_pays(x.numel() // x.size(-1), sum(sizes)) and not torch.compiler.is_compiling()
+        split = _split_pays(x.numel() // x.size(-1), sum(w.size(0) for w in ws)) and not torch.compiler.is_compiling()
         amp = torch.is_autocast_enabled("cuda")
         if torch.is_grad_enabled() and any(w.requires_grad for w in ws):
             # autocast's casts, made explicit for the autograd Function.  The split does not pay in the backward (dx
@@ -317,8 +321,8 @@ class MLA(nn.Module):
             dt = torch.get_autocast_dtype("cuda") if amp else \
                 torch.promote_types(torch.promote_types(ws[0].dtype, ws[1].dtype), ws[2].dtype)
             if (split or (dt == torch.bfloat16 and (amp or x.dtype == dt))) and training.plain_call(x, *ws):
-                return training.linear(x.to(dt), *ws, product=_down_product).split(sizes, dim=-1)
-            return torch.nn.functional.linear(x, torch.cat(ws, 0)).split(sizes, dim=-1)
+                return training.linear(x.to(dt), *ws, product=_down_product)
+            return torch.nn.functional.linear(x, torch.cat(ws, 0))
         dt = torch.get_autocast_dtype("cuda") if amp else ws[0].dtype
         key = tuple((w.data_ptr(), w._version) for w in ws) + (dt,)
         if getattr(self, "_down_key", None) != key:
@@ -326,10 +330,10 @@ class MLA(nn.Module):
             self._down_key = key
         W = self._down_w
         if not split:
-            return torch.nn.functional.linear(x, W).split(sizes, dim=-1)
+            return torch.nn.functional.linear(x, W)
         if torch.is_grad_enabled() and x.requires_grad:  # frozen weights, the input's gradient
-            return training.linear(x.to(W.dtype), W, product=_down_product).split(sizes, dim=-1)
-        return _linear_split_cols(x.to(W.dtype), W).split(sizes, dim=-1)
+            return training.linear(x.to(W.dtype), W, product=_down_product)
+        return _linear_split_cols(x.to(W.dtype), W)
 
     def _proj(self, name, x):
         """``self.<name>(x)``, with the weight gradient on this package's kernel where that is all the layer does."""
@@ -382,7 +386,12 @@ class MLA(nn.Module):
                                             q_content.dtype, appended, rows)
             q_content = ops.linear_rows(q_low.reshape(B * T, -1), Wq).view(B, T, -1)  # :208
         else:
-            q_low, qk_pos, kv_new = self._down_proj(x)  # :208-213, one GEMM (see _down_proj)
+            down = self._down_all(x)  # :208-213, one GEMM
+            if ROPE_FOLD and kv_cache is None and not use_cache and training.takes_attention(self, down):
+                cos, sin = self.rope.cos_cached, self.rope.sin_cached
+                return self._proj("o_proj", training.attention(self, down, cos, sin)), None
+            q_low, qk_pos, kv_new = down.split([self.q_down.weight.size(0), self.qk_rope.weight.size(0),
+                                                self.kv_down.weight.size(0)], dim=-1)
             q_content = self._proj("q_up", q_low)  # [B,T,H*dn]                   :208
         cdt = q_content.dtype
 

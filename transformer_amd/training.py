@@ -4,7 +4,11 @@
 library product, the weight gradient ``mla_weight_grad`` (transformer.py:208-213, :263, :300 under autograd).  Its sums
 reach fp32 weights as fp32: autocast's product rounds them to bf16 and casts them back.
 
-Callers take it only where nothing can tell the difference from ``nn.Linear`` (``takes``); everything else (tracing,
+``attention`` is everything between the down-projections' output and o_proj's input (transformer.py:208, :228-239,
+:306-315), as one Function whose backward writes each part of the down-projections' gradient where their product reads
+it.
+
+Callers take them only where nothing can tell the difference from ``nn.Linear`` (``takes``, ``takes_attention``); everything else (tracing,
 transforms, hooked or replaced submodules, other dtypes) keeps torch's own layers.
 """
 from __future__ import annotations
@@ -17,13 +21,8 @@ from . import kernels
 
 
 def plain_call(*tensors) -> bool:
-    """Whether an autograd.Function may stand in for torch's own operators: eager mode, no dispatch mode, functorch
-    transform or forward-mode level, and plain GPU tensors."""
-    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 \
-            or torch._C._functorch.peek_interpreter_stack() is not None \
-            or torch.autograd.forward_ad._current_level >= 0:
-        return False
-    return all((type(t) is torch.Tensor or type(t) is nn.Parameter) and t.is_cuda for t in tensors)
+    """Whether an autograd.Function may stand in for torch's own operators on ``tensors`` (see kernels.function_fits)."""
+    return kernels.function_fits(tensors)
 
 
 def plain_linear(m: nn.Module) -> bool:
@@ -38,13 +37,17 @@ def takes(m: nn.Module, x: torch.Tensor) -> bool:
     """Whether ``m(x)`` under autograd may run as ``linear``: a plain layer whose weight is trained, in bf16 arithmetic
     that torch's product accepts (autocast, or x in the weight's dtype)."""
     w = m._parameters.get("weight")
-    if w is None or not w.requires_grad or not torch.is_grad_enabled() or not plain_linear(m):
+    return (w is not None and w.requires_grad and torch.is_grad_enabled() and _bf16_arithmetic(m, x)
+            and plain_call(x, w))
+
+
+def _bf16_arithmetic(m: nn.Module, x: torch.Tensor) -> bool:
+    if not plain_linear(m):
         return False
+    w = m._parameters["weight"]
     if torch.is_autocast_enabled("cuda"):
-        ok = torch.get_autocast_dtype("cuda") == torch.bfloat16 and w.dtype in (torch.bfloat16, torch.float32)
-    else:
-        ok = w.dtype == torch.bfloat16 and x.dtype == w.dtype
-    return ok and plain_call(x, w)
+        return torch.get_autocast_dtype("cuda") == torch.bfloat16 and w.dtype in (torch.bfloat16, torch.float32)
+    return w.dtype == torch.bfloat16 and x.dtype == w.dtype
 
 
 def cat_weights(weights, dtype):
@@ -101,3 +104,98 @@ class _Linear(torch.autograd.Function):
 def linear(x: torch.Tensor, *weights, product=torch.nn.functional.linear) -> torch.Tensor:
     """``product(x, cat(weights))``, by default ``x @ cat(weights)^T``, in x's dtype; see the module."""
     return _Linear.apply(x, product, *weights)
+
+
+class _Attention(torch.autograd.Function):
+    """d [B, T, q_lora + (H + hr) 64 + d_latent], the down-projections' output -> o [B, T, H d_v].
+
+    The up-projections of the latent run as one product over [W_UK; W_UV], K and V the column views of its result.  In
+    the backward, dq_rope, dk_rope and the two products' results go straight to their columns of d's gradient, and dK
+    and dV to theirs of one buffer: one product gives the latent's gradient (dK W_UK + dV W_UV in one fp32 sum) and one
+    the weights'.  As separate nodes, autograd filled, copied, added and concatenated full-size tensors around them:
+    107 of 1495 us of a training pass of one block (default dims, B = 6, T = 2048)."""
+
+    @staticmethod
+    def forward(ctx, d, Wq, Wk, Wv, cos, sin, layout, scale):
+        H, dn, dv, hr, ql, dl = layout
+        with kernels.below_autograd():
+            B, T, n = d.shape
+            d2 = d.reshape(B * T, n)
+            Wqb, Wkv = cat_weights((Wq,), d.dtype), cat_weights((Wk, Wv), d.dtype)
+            qk = d2[:, ql:n - dl].view(B, T, H + hr, 64)
+            q = torch.mm(d2[:, :ql], Wqb.t()).view(B, T, H, dn)
+            kv = torch.mm(d2[:, n - dl:], Wkv.t())
+            k_nope, v = _kv_views(kv, B, T, H, dn, dv)
+            k_rope = kernels.eager.rope(qk[:, :, H:], cos, sin, 0, False)
+            o, lse, q_rot = kernels.eager.prefill_fwd_rope(q, qk[:, :, :H], k_nope, k_rope, v, cos, sin, scale, True, 0,
+                                                           0, True)
+        ctx.save_for_backward(d, Wqb, Wkv, q, q_rot, kv, k_rope, o, lse, cos, sin)
+        ctx.weights, ctx.layout, ctx.scale = (Wq, Wk, Wv), layout, scale
+        return o.view(B, T, H * dv)
+
+    @staticmethod
+    def backward(ctx, do):
+        d, Wqb, Wkv, q, q_rot, kv, k_rope, o, lse, cos, sin = ctx.saved_tensors
+        H, dn, dv, hr, ql, dl = ctx.layout
+        B, T, n = d.shape
+        if torch.is_grad_enabled():  # the backward is itself differentiated: through the operators
+            inputs = [t for t, need in zip((d, *ctx.weights), ctx.needs_input_grad) if need]
+            with torch.enable_grad():
+                out = _attention_by_operators(d, *ctx.weights, cos, sin, ctx.layout, ctx.scale)
+            got = iter(torch.autograd.grad(out, inputs, do, create_graph=True))
+            return tuple(next(got) if need else None for need in ctx.needs_input_grad[:4]) + (None,) * 4
+        d2 = d.reshape(B * T, n)
+        dd = torch.empty(B * T, n, dtype=d.dtype, device=d.device)
+        dqk = dd[:, ql:n - dl].view(B, T, H + hr, 64)
+        dq = torch.empty(B, T, H, dn, dtype=d.dtype, device=d.device)
+        dkv = torch.empty_like(kv)
+        dk_nope, dvv = _kv_views(dkv, B, T, H, dn, dv)
+        k_nope, v = _kv_views(kv, B, T, H, dn, dv)
+        kernels._prefill_bwd_impl(do.reshape(B, T, H, dv), q, q_rot, k_nope, k_rope, v, o, lse, ctx.scale, True, 0, cos,
+                                  sin, 0, out=(dq, dqk[:, :, :H], dk_nope, dqk[:, :, H:], dvv))
+        kernels.eager.rope_(dqk[:, :, H:], cos, sin, 0, True)
+        dq2 = dq.view(B * T, H * dn)
+        if ctx.needs_input_grad[0]:
+            torch.mm(dq2, Wqb, out=dd[:, :ql])
+            torch.mm(dkv, Wkv, out=dd[:, n - dl:])
+        (Wq, Wk, Wv), (_, nq, nk, nv) = ctx.weights, ctx.needs_input_grad[:4]
+        (gq,) = weight_grads(dq2, d2[:, :ql], (Wq,), (nq,))
+        gk, gv = weight_grads(dkv, d2[:, n - dl:], (Wk, Wv), (nk, nv))
+        return dd.view(B, T, n) if ctx.needs_input_grad[0] else None, gq, gk, gv, None, None, None, None
+
+
+def _kv_views(kv, B, T, H, dn, dv):
+    """K_nope [B, T, H, dn] and V [B, T, H, dv] in the columns of ``kv [B T, H (dn + dv)]``."""
+    return kv[:, :H * dn].view(B, T, H, dn), kv[:, H * dn:].view(B, T, H, dv)
+
+
+def _attention_by_operators(d, Wq, Wk, Wv, cos, sin, layout, scale):
+    H, dn, dv, hr, ql, dl = layout
+    B, T, n = d.shape
+    q_low, qk, kv = d.split([ql, (H + hr) * 64, dl], -1)
+    lin = torch.nn.functional.linear
+    qk = qk.view(B, T, H + hr, 64)
+    q, k, v = (lin(t, w.to(d.dtype)).view(B, T, H, -1) for t, w in ((q_low, Wq), (kv, Wk), (kv, Wv)))
+    k_rope = kernels.eager.rope(qk[:, :, H:], cos, sin, 0, False)
+    o, _, _ = kernels.eager.prefill_fwd_rope(q, qk[:, :, :H], k, k_rope, v, cos, sin, scale, True, 0, 0, True)
+    return o.reshape(B, T, H * v.size(-1))
+
+
+def takes_attention(mla, d: torch.Tensor) -> bool:
+    """Whether ``attention`` may run the no-cache branch on the down-projections' bf16 output ``d``: its gradient or a
+    weight's is needed, the three layers are plain in bf16 arithmetic, and every part of ``d`` is whole 16-byte runs."""
+    mods = [mla._modules[n] for n in ("q_up", "k_up", "v_up")]
+    if not (torch.is_grad_enabled() and d.dtype == torch.bfloat16 and d.numel() > 0
+            and mla.d_latent % 8 == 0 and mods[0].in_features % 8 == 0
+            and mla.content_dim in kernels.SUPPORTED_NOPE and mla.v_head_dim in kernels.SUPPORTED_V):
+        return False
+    ws = [m._parameters.get("weight") for m in mods]
+    return (all(w is not None for w in ws) and (d.requires_grad or any(w.requires_grad for w in ws))
+            and all(_bf16_arithmetic(m, d) for m in mods) and plain_call(d, *ws))
+
+
+def attention(mla, d: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+    """o_proj's input from the down-projections' output, causal over its own positions; see ``_Attention``."""
+    q, k, v = (mla._modules[n].weight for n in ("q_up", "k_up", "v_up"))
+    layout = (mla.n_heads, mla.content_dim, mla.v_head_dim, mla.n_k_rope_heads, q.size(1), mla.d_latent)
+    return _Attention.apply(d, q, k, v, cos, sin, layout, mla.scale)
