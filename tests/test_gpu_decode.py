@@ -281,3 +281,38 @@ def test_decode_out_writes_a_caller_ctx(ops, B, L, splits):
     torch.cuda.synchronize()
     assert torch.equal(out, out_ref) and torch.equal(lse, lse_ref), "out / lse differ from the op's"
     assert torch.equal(ctx, ctx_ref) and torch.equal(lse, lse_dec), "ctx / lse differ from mla_decode's"
+
+
+@pytest.mark.parametrize("B,H,L,DL,splits", [
+    (1, 2, 1, 64, 0),        # one row: every lane repeats it
+    (2, 8, 15, 128, 1),      # a ragged only tile; one half of the heads
+    (1, 9, 65, 512, 1),      # a fifth tile (the first wave's second), one head in the second half
+    (2, 16, 209, 256, 2),    # tiles that do not divide the four waves
+    (1, 33, 150, 384, 1),    # three head groups, the last of one head
+    (3, 14, 2000, 384, 0),   # the reference's default heads over many splits
+])
+def test_decode_per_head_rope_matches_oracle(ops, B, H, L, DL, splits):
+    print(f"case per-head k_rope B={B} H={H} L={L} DL={DL} splits={splits}", flush=True)
+    g = torch.Generator().manual_seed(H * L + DL)
+    q_lat, q_rope, c, _ = make(B, H, L, DL, 1, seed=L + DL)
+    kr = randn_bf16((B, L, H + 1, 64), g)[:, :, :H].transpose(1, 2)  # strided heads, as a fused projection leaves them
+    scale = 1 / math.sqrt(128)
+    ctx, lse = run(ops, q_lat, q_rope, c, kr, scale, splits=splits)
+    rc, rl = oracle(q_lat, q_rope, c, kr, scale)
+    check_close(ctx.double(), rc, "ctx")
+    torch.testing.assert_close(lse.double(), rl, rtol=0, atol=1e-3)
+    ctx2, lse2 = run(ops, q_lat, q_rope, c, kr, scale, splits=splits)
+    assert torch.equal(ctx, ctx2) and torch.equal(lse, lse2)
+
+
+def test_decode_per_head_rope_keeps_a_heads_nan_to_it(ops):
+    B, H, L, DL = 1, 14, 100, 384
+    q_lat, q_rope, c, kr = make(B, H, L, DL, H, seed=5)
+    clean, _ = run(ops, q_lat, q_rope, c, kr, 0.1)
+    kr[0, 6, 37, 5], kr[0, 11, 70, 60] = float("nan"), float("inf")
+    ctx, _ = run(ops, q_lat, q_rope, c, kr, 0.1)
+    same = [h for h in range(H) if h not in (6, 11)]
+    # (an infinite score makes the wave rescale at that tile, so the others' bf16 P is rounded about another maximum:
+    # each of at most 100 terms moves by 2^-8, which the parity bound of the oracle tests covers)
+    check_close(ctx[0, same].double(), clean[0, same].double(), "other heads")
+    assert ctx[0, 6].isnan().all()

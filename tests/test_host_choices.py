@@ -193,3 +193,13 @@ def test_training_layers_take_only_plain_linears():
     assert training.plain_linear(lin)
     torch.nn.utils.parametrizations.weight_norm(lin)
     assert not training.plain_linear(lin)
+
+
+def test_rows_path_takes_the_projections_where_only_the_absorption_does_not_fit():
+    # the reference's default dims: W_UK's K = 64 is outside linear_rows, the projections are inside
+    from transformer_amd import MLA, ModelArgs
+    m = MLA(ModelArgs(max_seq_len=64)).to(torch.bfloat16)
+    x = torch.zeros(4, 1, m.d_model, dtype=torch.bfloat16)
+    with torch.no_grad():
+        assert m._rows_proj_ok() and not m._rows_dims_ok() and m._rows_path(x)
+        assert not m._rows_path(torch.zeros(65, 1, m.d_model, dtype=torch.bfloat16))

@@ -15,7 +15,8 @@
 //   * the next tile is prefetched into registers while the current one is in the
 //     wave's private LDS buffer (no workgroup barrier in the loop);
 //   * S^T [16 tok][16 heads] = C [16 tok][KW] . Q^T     v_mfma_f32_16x16x32_bf16, the
-//     shared k_rope being 64 more columns of the row (KW = DL + 64);
+//     shared k_rope being 64 more columns of the row (KW = DL + 64); per-head k_rope rows
+//     go straight to registers as operands of their own (load_rope below);
 //   * online softmax per head inside the wave (lane = head, registers = tokens);
 //   * O^T [DL][16 heads] += C^T [DL][16 tok] . P^T [16 tok][16 heads]
 //     (v_mfma_f32_16x16x16_bf16): C^T comes from ds_read_b64_tr_b16 (the LDS transpose
@@ -34,6 +35,7 @@
 // (16 tokens x one chunk) and the transpose reads (4 tokens x 2 chunks per 16 lanes)
 // free of bank conflicts.
 #include <mutex>
+#include <type_traits>
 
 #include "mla_common.h"
 
@@ -94,7 +96,7 @@ __global__ __launch_bounds__(256, 1) void decode_kernel(DecParams p) {
   using C = DecCfg<DL, SHARED>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS];
   __shared__ __attribute__((aligned(16))) unsigned char qs[16 * C::RS * 16];
-  __shared__ __attribute__((aligned(16))) unsigned char qrs[SHARED ? 16 : 16 * 9 * 16];
+  __shared__ __attribute__((aligned(16))) unsigned char qrs[SHARED ? 16 : 16 * 8 * 16];
   __shared__ float m_s[4][16], l_s[4][16];
 
   int unit, split;
@@ -166,9 +168,50 @@ __global__ __launch_bounds__(256, 1) void decode_kernel(DecParams p) {
     }
   };
 
+  // Per-head k_rope (DL + 16 x 64 columns a token, most of them k_rope): a head's 16 rows of the tile are the A operand
+  // of two MFMAs as they lie (row l16, 16-byte chunk 4 ks + G), read as 64-byte runs straight into registers.  Heads past
+  // H repeat the last one.  The heads come in two halves through one set of registers: the first half's rows of the next
+  // tile are in flight over the end of a tile, the second half's over its latent scores, with the next latent rows
+  // issued after them, so no wait includes a later load (a set of registers for each half was 8 % slower).
+  // Lane (head, 4 tokens) reading its own rows at the point of use, 64 rows of 16 bytes a load and nothing in flight
+  // before, took 40.8 us with its merge at B = 16 over 2500 tokens (14 heads, d_latent 384, 102 MB) and 26.2 at B = 1
+  // over 1000; whole rows and VALU dot products 34.9 and 23.2; this takes 33.8 and 24.2 (75.1 against 88.5
+  // at B = 32 over 4096, 44.3 against 53.0 at B = 8 over 7000).
+  constexpr int NKR = SHARED ? 1 : 16;
+  u32x4 krp[NKR];
+  auto load_rope = [&](int t0, int half) {
+    int t = t0 + l16;
+    t = t < Lb ? t : Lb - 1;
+    const bf16* row = kr_b + (int64_t)t * p.k_rope_st + 8 * G;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const bf16* r = row + (int64_t)min(hg * 16 + 8 * half + j, p.H - 1) * p.k_rope_sh;
+      krp[2 * j] = ldg16(r);
+      krp[2 * j + 1] = ldg16(r + 32);
+    }
+  };
+  // rope scores of a half, into rsc (the layout of S^T): every column of B is the head's q_rope, so every lane gets its
+  // tokens' scores of that head and lane l16 keeps head l16's.  (One chain over the heads, each with the other heads'
+  // columns zero, would carry a head's infinities into the others as NaN.)
+  auto score_rope = [&](int half, f32x4& rsc) {
+    int qoff = 1024 * half + 16 * G;
+    asm volatile("" : "+v"(qoff));  // read at use: hoisted out of the loop, q_rope would take 128 registers
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      f32x4 d = mfma16(as_bf16x8(krp[2 * j]), as_bf16x8(lds16(qrs + qoff + j * 128)), f32x4{0.f, 0.f, 0.f, 0.f});
+      d = mfma16(as_bf16x8(krp[2 * j + 1]), as_bf16x8(lds16(qrs + qoff + j * 128 + 64)), d);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rsc[r] = l16 == 8 * half + j ? d[r] : rsc[r];
+      if (j & 1) __builtin_amdgcn_sched_barrier(0);  // two heads' q_rope live at a time, not all eight's
+    }
+  };
+
   // the first tile is in flight while Q is staged
   int k = w;
-  if (k < n_tiles) load_tile(t_begin + k * C::TT);
+  if (k < n_tiles) {
+    load_tile(t_begin + k * C::TT);
+    if constexpr (!SHARED) load_rope(t_begin + k * C::TT, 0);
+  }
 
   // ---- Q^T (B operand of S^T = C . Q^T: column = head, K slot = dim 32 ks + 8 G + e) is
   // staged once in LDS with the tile swizzle (row = head); per-head q_rope rows too.
@@ -195,7 +238,7 @@ __global__ __launch_bounds__(256, 1) void decode_kernel(DecParams p) {
   if (k < n_tiles) {
     store_tile();
     staged = true;
-    if (k + 4 < n_tiles) load_tile(t_begin + (k + 4) * C::TT);
+    if (SHARED && k + 4 < n_tiles) load_tile(t_begin + (k + 4) * C::TT);
   }
 #pragma unroll
   for (int i = 0; i < QCH; ++i) {
@@ -212,7 +255,7 @@ __global__ __launch_bounds__(256, 1) void decode_kernel(DecParams p) {
       const int hh = hg * 16 + hr;
       const u32x4 v = hh < p.H ? ldg16(p.q_rope + (int64_t)b * p.q_rope_sb + (int64_t)hh * p.q_rope_sh + 8 * c)
                                : u32x4{0u, 0u, 0u, 0u};
-      sts16(qrs + (hr * 9 + c) * 16, v);
+      sts16(qrs + (hr * 8 + c) * 16, v);
     }
   }
   __syncthreads();
@@ -237,11 +280,20 @@ __global__ __launch_bounds__(256, 1) void decode_kernel(DecParams p) {
   float m_run = -INFINITY;  // log2-domain running max of head h (same in the 4 lane groups)
   float l_part = 0.f;       // this lane's share of the running sum (its 4 tokens per tile)
 
-  for (; k < n_tiles; k += 4) {
+  // one tile; `more`: the wave has a next one, whose loads are issued here
+  auto tile = [&](auto more) {
     const int t0 = t_begin + k * C::TT;
-    if (!staged) {
-      store_tile();
-      if (k + 4 < n_tiles) load_tile(t0 + 4 * C::TT);
+    [[maybe_unused]] f32x4 rsc = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (SHARED) {
+      if (!staged) {
+        store_tile();
+        if (k + 4 < n_tiles) load_tile(t0 + 4 * C::TT);
+      }
+    } else {
+      if (!staged) store_tile();
+      score_rope(0, rsc);
+      load_rope(t0, 1);
+      if (more) load_tile(t0 + 4 * C::TT);
     }
     staged = false;
 
@@ -252,25 +304,10 @@ __global__ __launch_bounds__(256, 1) void decode_kernel(DecParams p) {
       const int off = ((ks & 1) ? offA1 : offA0) + (ks >> 1) * 128;
       sacc = mfma16(as_bf16x8(lds16(buf + off)), as_bf16x8(lds16(qs + off)), sacc);
     }
-    if (!SHARED) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        int t = t0 + 4 * G + r;
-        t = t < Lb ? t : Lb - 1;
-        const bf16* kr = kr_b + (int64_t)(h_ok ? h : 0) * p.k_rope_sh + (int64_t)t * p.k_rope_st;
-        float acc = 0.f;
-#pragma unroll
-        for (int c8 = 0; c8 < 8; ++c8) {
-          const u32x4 v = ldg16(kr + 8 * c8);
-          const u32x4 qv = lds16(qrs + (l16 * 9 + c8) * 16);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            acc += lo_bf16(v[e]) * lo_bf16(qv[e]);
-            acc += hi_bf16(v[e]) * hi_bf16(qv[e]);
-          }
-        }
-        sacc[r] += acc;
-      }
+    if constexpr (!SHARED) {
+      score_rope(1, rsc);
+      if (more) load_rope(t0 + 4 * C::TT, 0);
+      sacc += rsc;
     }
 
     // online softmax of head l16 over this tile's 16 tokens
@@ -313,6 +350,13 @@ __global__ __launch_bounds__(256, 1) void decode_kernel(DecParams p) {
       const s16x4 bv = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(buf + off));
       oacc[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bv, pa, oacc[nb], 0, 0, 0);
     }
+  };
+  if constexpr (SHARED) {
+    for (; k < n_tiles; k += 4) tile(std::true_type{});  // (asks k itself)
+  } else {
+    // the last tile apart: loads under a condition inside the loop made the compiler hold two copies of krp (spills)
+    for (; k + 4 < n_tiles; k += 4) tile(std::true_type{});
+    if (k < n_tiles) tile(std::false_type{});
   }
 
   // ---- merge the 4 waves: M = max_w m_w, O = sum_w 2^(m_w - M) O_w, L likewise

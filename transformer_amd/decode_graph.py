@@ -134,8 +134,10 @@ class DecodeGraph:
         # q_up, W_UK transposed per head [H, DL, dn] (the absorption as H products) and o_proj
         # (the module's own choice for this batch: autograd off, bf16, at most ROWS_FAST_M rows and
         # every product within the kernel's shape limits)
-        self.rows = cdt == torch.bfloat16 and mla._rows_dims_ok() and B <= kernels.ROWS_FAST_M
-        if self.rows:
+        self.rows = cdt == torch.bfloat16 and mla._rows_proj_ok() and B <= kernels.ROWS_FAST_M
+        # the absorption on absorb_q where K = d_nope does not fit linear_rows
+        self.rows_uk = self.rows and kernels.rows_fit(dn, DL)
+        if self.rows_uk:
             self.w_ukt = self.w_uk.transpose(1, 2).contiguous()
 
         # warm up on a side stream (library handles and allocator pools), then record; the
@@ -179,7 +181,7 @@ class DecodeGraph:
                                      self.k_rope, cos, sin, pos, self.seq_lens, 0, H, pos_next)
         seq_lens = self.seq_lens
         # absorbed decode (:249-291)
-        if self.rows:
+        if self.rows_uk:
             q_lat = ops.linear_rows(q_content.view(B, H, dn), self.w_ukt)  # [B,H,DL] (:252-254)
         else:
             q_lat = ops.absorb_q(q_content.view(B, H, dn).to(torch.bfloat16), self.w_uk)

@@ -286,15 +286,20 @@ class MLA(nn.Module):
     def _rows_dims_ok(self):
         """Whether every product of the decode step fits linear_rows' shape limits (K a
         multiple of 128 up to ROWS_MAX_K, N a multiple of 4)."""
+        return self._rows_proj_ok() and kernels.rows_fit(self.content_dim, self.d_latent)
+
+    def _rows_proj_ok(self):
+        """Whether the decode step's projections fit linear_rows.  The W_UK absorption may not (K = 64 at the
+        reference's default dims): it then runs on absorb_q between them."""
         H, dn, dv = self.n_heads, self.content_dim, self.v_head_dim
         n_down = self.q_down.weight.size(0) + self.qk_rope.weight.size(0) + self.kv_down.weight.size(0)
         return all(kernels.rows_fit(K, N) for K, N in (
-            (self.d_model, n_down), (self.q_up.weight.size(1), H * dn), (dn, self.d_latent), (H * dv, self.d_model)))
+            (self.d_model, n_down), (self.q_up.weight.size(1), H * dn), (H * dv, self.d_model)))
 
     def _rows_path(self, x):
         """Few-row bf16 products (the decode step): autograd off, at most ROWS_FAST_M rows, and
         bf16 arithmetic (bf16 weights, or bf16 autocast)."""
-        if torch.is_grad_enabled() or x.size(0) * x.size(1) > kernels.ROWS_FAST_M or not self._rows_dims_ok():
+        if torch.is_grad_enabled() or x.size(0) * x.size(1) > kernels.ROWS_FAST_M or not self._rows_proj_ok():
             return False
         if torch.is_autocast_enabled("cuda"):
             return torch.get_autocast_dtype("cuda") == torch.bfloat16
@@ -464,7 +469,7 @@ class MLA(nn.Module):
         b = self._bf16
         if T == 1:
             # absorbed decode (:249-291): q_lat = q_nope W_UK, ctx = softmax(s) c_kv, out = ctx W_UV^T
-            if rows:
+            if rows and kernels.rows_fit(dn, self.d_latent):
                 # W_UK transposed per head [H, DL, dn], so the absorption is H few-row products
                 Wkt = self._cached_weight("k_up:t", lambda: self.k_up.weight.view(H, dn, self.d_latent).transpose(1, 2),
                                           torch.bfloat16)
