@@ -120,3 +120,24 @@ def test_norm_linear_rejects_bad_shapes(ops):
     with pytest.raises(TypeError):
         ops.norm_linear(x.float(), torch.zeros(8, 64, dtype=torch.bfloat16, device="cuda"), torch.ones(64, device="cuda"),
                         1e-6)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (6391, 2600, 32),   # 256 x 256 tiles beside a 40-column remainder's tiles; one stage
+    (6391, 2600, 128),  # the ring's four stages
+    (6391, 2600, 160),  # five: one through the steady loop
+    (6391, 2500, 96),   # 256 x 256 tiles, the last column of them ragged
+    (2735, 2000, 512),  # 256 x 128 tiles, ragged both ways
+    (1100, 1304, 544),  # 128 x 128 tiles, ragged both ways
+])
+def test_norm_linear_tile_shapes(ops, M, N, K):
+    print(f"case M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).bfloat16()
+    w_norm = torch.rand(K, generator=g, device="cuda") + 0.5
+    y, r = ops.norm_linear(x, w, w_norm, 1e-6)
+    check_r(r, x.cpu(), 1e-6)
+    xn = ((x.float() * r[:, None]) * w_norm).to(torch.bfloat16)
+    within_one_ulp(y, xn.double() @ w.double().t().contiguous(), f"M={M} N={N} K={K}")
+    assert torch.equal(y, ops.norm_linear(x, w, w_norm, 1e-6)[0])
