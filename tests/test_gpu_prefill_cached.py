@@ -160,3 +160,20 @@ def test_prefill_cached_is_deterministic(ops):
     a = ops.prefill_cached(q_lat, q_rope, c, kr, 680, SCALE)
     b = ops.prefill_cached(q_lat, q_rope, c, kr, 680, SCALE)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("B,T,H,L0,DL", [
+    (1, 119, 16, 1500, 512),  # 8 waves with key ranges: 15 query blocks, the last ragged
+    (3, 100, 16, 700, 128),   # ranges whose workgroups stay within one round
+    (2, 70, 20, 900, 384),    # two head groups
+    (1, 5, 16, 4100, 256),    # few queries over many ranges
+])
+def test_prefill_cached_chosen_workgroups_and_ranges(ops, B, T, H, L0, DL):
+    print(f"case B={B} T={T} H={H} L0={L0} DL={DL}", flush=True)
+    q_lat, q_rope, c, kr = make(B, T, H, L0 + T, DL, seed=L0 + T)
+    ctx, lse = run(ops, q_lat, q_rope, c, kr, L0)
+    rc, rl = oracle(q_lat, q_rope, c, kr, L0, T)
+    check_close(ctx.double(), rc, "ctx")
+    torch.testing.assert_close(lse.double(), rl, rtol=0, atol=1e-3)
+    ctx2, lse2 = run(ops, q_lat, q_rope, c, kr, L0)
+    assert torch.equal(ctx, ctx2) and torch.equal(lse, lse2)

@@ -471,10 +471,16 @@ __global__ __launch_bounds__(256) void prefill_cached_merge_wide_kernel(PcParams
   if (p.lse && lane == 0) p.lse[((int64_t)b * p.H + h) * p.T + t] = L > 0.f ? (M + fast_log2(L)) * kLn2 : -INFINITY;
 }
 
-// workgroups of 8 waves (8 queries) share each tile among more queries; when they would not
-// fill the chip's 256 CUs, workgroups of 4 waves give twice as many, and if those still do not,
-// the keys are split into ranges of at least kPcMinSplitTiles tiles until they do
-constexpr int kPcBigNW = 8, kPcSmallNW = 4, kPcFillWgs = 256, kPcMinSplitTiles = 4, kPcMaxSplits = 256;
+// Workgroups of 8 waves (8 queries) share each tile among more queries and run two waves per SIMD; workgroups of 4 give
+// twice as many, and key ranges multiply either (at least kPcMinSplitTiles tiles each).  The pair of least estimated time
+// is taken, for up to kPcRounds rounds of 256 workgroups (one per CU: the tile ring takes 110 KB at d_latent 512):
+//   rounds x (tiles of a range x time per tile + 6 us) + the merge (2 us + its fp32 partials at 3.6 MB a us),
+// with 1.68 (4 waves) and 2.35 us (8) per tile at d_latent 512, fitted to graph-replayed calls (16 heads, 4 / 8 waves):
+// B = 8, T = 64 over 4000 keys 125.0 / 101.3 us (2 and 4 ranges), B = 1 34.4 / 40.2, B = 4, T = 128 over 1024 50.5 / 52.2,
+// B = 16, T = 16 over 2000 43.8 / 48.3.  Always 4 waves below 256 workgroups of 8, and ranges to reach at least 256
+// workgroups, started a nearly empty second round: B = 3, T = 100 over 2000 77.0 us (300 workgroups), now 54.7; B = 16,
+// T = 100 over 1000 117.7 us (400), now 90.5; B = 5, T = 64 over 7000 190 us, now 114.
+constexpr int kPcBigNW = 8, kPcSmallNW = 4, kPcFillWgs = 256, kPcMinSplitTiles = 4, kPcMaxSplits = 256, kPcRounds = 4;
 
 struct PcLayout {
   int nw = 0, n_hg = 0, n_qb = 0, S = 1, chunk_tiles = 0;
@@ -485,16 +491,33 @@ struct PcLayout {
 static PcLayout pc_layout(const mla_prefill_cached_args* a) {
   PcLayout d;
   d.n_hg = (int)((a->H + 15) / 16);
-  const int64_t n_wg_big = a->B * (int64_t)d.n_hg * ((a->T + kPcBigNW - 1) / kPcBigNW);
-  d.nw = n_wg_big < kPcFillWgs ? kPcSmallNW : kPcBigNW;
-  d.n_qb = (int)((a->T + d.nw - 1) / d.nw);
-  d.n_wg = a->B * (int64_t)d.n_hg * d.n_qb;
   const int64_t n_tiles = (a->L0 + a->T + 31) / 32;  // tiles of the workgroup that sees the most keys
+  const auto n_wg = [&](int nw) { return a->B * (int64_t)d.n_hg * ((a->T + nw - 1) / nw); };
   int64_t S = a->num_splits;
-  if (S <= 0)
-    S = d.n_wg >= kPcFillWgs ? 1
-                             : std::min<int64_t>((kPcFillWgs + d.n_wg - 1) / d.n_wg,
-                                                 std::max<int64_t>(1, n_tiles / kPcMinSplitTiles));
+  if (S > 0) {
+    d.nw = n_wg(kPcBigNW) < kPcFillWgs ? kPcSmallNW : kPcBigNW;
+  } else {
+    const double per_tile = (double)(2 * a->d_latent + 64) / 1088.0;  // of the time at d_latent 512
+    const double part = (double)a->B * d.n_hg * a->T * 16.0 * a->d_latent * 4.0 / 3.6e6;  // us per range merged
+    const int64_t most = std::min<int64_t>(std::max<int64_t>(1, n_tiles / kPcMinSplitTiles), kPcMaxSplits);
+    double best = 1e300;
+    for (int nw : {kPcSmallNW, kPcBigNW}) {
+      for (int r = 1; r <= kPcRounds; ++r) {
+        const int64_t want = std::min<int64_t>(std::max<int64_t>(1, (int64_t)r * kPcFillWgs / n_wg(nw)), most);
+        const int64_t tiles = (n_tiles + want - 1) / want, s = (n_tiles + tiles - 1) / tiles;
+        const double rounds = (double)((n_wg(nw) * s + kPcFillWgs - 1) / kPcFillWgs);
+        const double t = rounds * ((double)tiles * (nw == kPcSmallNW ? 1.68 : 2.35) * per_tile + 6.0) +
+                         (s > 1 ? 2.0 + part * (double)s : 0.0);
+        if (t < best) {
+          best = t;
+          d.nw = nw;
+          S = s;
+        }
+      }
+    }
+  }
+  d.n_qb = (int)((a->T + d.nw - 1) / d.nw);
+  d.n_wg = n_wg(d.nw);
   S = std::max<int64_t>(1, std::min<int64_t>({S, n_tiles, (int64_t)kPcMaxSplits}));
   const int64_t chunk = (n_tiles + S - 1) / S;
   d.S = (int)((n_tiles + chunk - 1) / chunk);  // no empty trailing range
