@@ -27,7 +27,8 @@
 //   dQ kernel, wave = 32 queries, loop over 32-key blocks (K, V in LDS):
 //     S^T (32k x 32q) = K . Q^T,  dP^T = V . dO^T   (lanes own a query)
 //     dQ^T (DQK x 32q) += K^T . dS^T                (K^T by transpose read)
-// Workgroups take mirrored pairs of tiles of one (b, h) so causal work is balanced.
+// Workgroups take mirrored pairs of tiles of one (b, h) so causal work is balanced, or single tiles, longest first, where
+// pairs would leave much of a last round empty (TileGrid in mla_common.h).
 #include <type_traits>
 
 #include "mla_common.h"
@@ -46,6 +47,7 @@ struct BwdParams {
   int ds_e;        // (31 + max(q_offset, 0)) / 32: the causal rows' extra visible key blocks
   int64_t ds_bh_blocks;  // stored blocks per (b, h)
   int B, H, Tq, Tk;
+  int single_kt, single_qt;  // one key (query) tile per workgroup, longest first, instead of mirrored pairs (TileGrid)
   int shared_rope;
   mla_strides do_s, qn_s, qr_s, kn_s, kr_s, v_s, o_s;
   mla_strides dqn_s, dqr_s, dkn_s, dkr_s, dv_s;
@@ -158,10 +160,20 @@ __device__ __forceinline__ int ds_prefix32(int Q, int nkb, int e, bool causal) {
   return (int)(((unsigned)m * (unsigned)(m + 1)) >> 1) + m * e + (Q - m) * nkb;
 }
 
-// workgroup id -> (b, h, the pair of tiles r and n - 1 - r of that (b, h)); XCD-contiguous
-__device__ __forceinline__ void bwd_coords(int n_tiles, int H, int& b, int& h, int& ta, int& tb, int& n_items) {
+// workgroup id -> (b, h, the pair of tiles r and n - 1 - r of that (b, h)), XCD-contiguous; or one tile of it
+__device__ __forceinline__ void bwd_coords(int n_tiles, int H, int n_bh, int single, int& b, int& h, int& ta, int& tb,
+                                           int& n_items) {
   const int n = gridDim.x;
   int id = blockIdx.x;
+  if (single) {  // one tile each, tile 0's end of the mirror first; (b, h) fastest
+    ta = id / n_bh;
+    tb = n_tiles - 1 - ta;
+    n_items = 1;
+    const int bh1 = id - ta * n_bh;
+    b = bh1 / H;
+    h = bh1 - b * H;
+    return;
+  }
   if ((n & 7) == 0) id = (id & 7) * (n >> 3) + (id >> 3);
   const int n_pairs = (n_tiles + 1) >> 1;
   const int bh = id / n_pairs;
@@ -267,7 +279,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdParams p) {
 
   const int n_kt = (p.Tk + C::BKV - 1) / C::BKV;
   int b, h, kt_a, kt_b, n_items;
-  bwd_coords(n_kt, p.H, b, h, kt_a, kt_b, n_items);
+  bwd_coords(n_kt, p.H, p.B * p.H, p.single_kt, b, h, kt_a, kt_b, n_items);
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   __builtin_assume(wv >= 0 && wv < 8);
@@ -653,7 +665,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p) {
 
   const int n_qt = (p.Tq + C::BQQ - 1) / C::BQQ;
   int b, h, qt_a, qt_b, n_items;
-  bwd_coords(n_qt, p.H, b, h, qt_b, qt_a, n_items);  // qt_a: the longer tile first
+  bwd_coords(n_qt, p.H, p.B * p.H, p.single_qt, b, h, qt_b, qt_a, n_items);  // qt_a: the longer tile first
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   __builtin_assume(w >= 0 && w < 4);
@@ -972,7 +984,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_ds_kernel(BwdParams p) {
 
   const int n_qt = (p.Tq + C::BQQ - 1) / C::BQQ;
   int b, h, qt_a, qt_b, n_items;
-  bwd_coords(n_qt, p.H, b, h, qt_b, qt_a, n_items);  // qt_a: the longer tile first
+  bwd_coords(n_qt, p.H, p.B * p.H, p.single_qt, b, h, qt_b, qt_a, n_items);  // qt_a: the longer tile first
   {
     // (b, h) in reverse order: the dK/dV pass walks each XCD's share of (b, h) upwards, so
     // the first workgroups here read the blocks it stored last, which may still sit in the
@@ -1242,7 +1254,7 @@ __global__ __launch_bounds__(256) void bwd_dkrope_reduce_kernel(BwdParams p) {
 }
 
 template <int DN>
-static int launch_bwd(const BwdParams& prm, hipStream_t s) {
+static int launch_bwd(BwdParams prm, hipStream_t s) {
   // every grid is checked before the first launch, so a rejected call does no work
   const int64_t n_rec = (int64_t)prm.B * prm.H * ((prm.Tq + 31) / 32);  // 32-query records
   const int64_t n_kt = (prm.Tk + DkdvCfg<DN>::BKV - 1) / DkdvCfg<DN>::BKV;
@@ -1252,11 +1264,15 @@ static int launch_bwd(const BwdParams& prm, hipStream_t s) {
                 (int64_t)prm.B * prm.H * n_qt < (1ll << 31) && (n_rope + 255) / 256 < (1ll << 31),
             MLA_ERR_INVALID_ARG, "mla_prefill_bwd: grid too large");
   if (n_rec > 0) bwd_rowdot_kernel<<<dim3((unsigned)n_rec), dim3(256), 0, s>>>(prm);
-  bwd_dkdv_kernel<DN><<<dim3((unsigned)(prm.B * prm.H * ((n_kt + 1) / 2))), dim3(512), 0, s>>>(prm);
-  if (prm.ds_ws)
-    bwd_dq_ds_kernel<DN><<<dim3((unsigned)(prm.B * prm.H * ((n_qt + 1) / 2))), dim3(256), 0, s>>>(prm);
-  else
-    bwd_dq_kernel<DN><<<dim3((unsigned)(prm.B * prm.H * ((n_qt + 1) / 2))), dim3(256), 0, s>>>(prm);
+  const int64_t n_bh = (int64_t)prm.B * prm.H;
+  const bool square = prm.causal && prm.q_offset == 0;
+  prm.single_kt = single_tiles_one_per_cu(TileGrid{n_bh, n_kt, square});  // 8-wave workgroups, one per CU
+  prm.single_qt = single_tiles_two_per_cu(TileGrid{n_bh, n_qt, square});
+  const dim3 kt_grid((unsigned)(n_bh * (prm.single_kt ? n_kt : (n_kt + 1) / 2)));
+  const dim3 qt_grid((unsigned)(n_bh * (prm.single_qt ? n_qt : (n_qt + 1) / 2)));
+  bwd_dkdv_kernel<DN><<<kt_grid, dim3(512), 0, s>>>(prm);
+  if (prm.ds_ws) bwd_dq_ds_kernel<DN><<<qt_grid, dim3(256), 0, s>>>(prm);
+  else bwd_dq_kernel<DN><<<qt_grid, dim3(256), 0, s>>>(prm);
   if (n_rope > 0 && !prm.ds_ws)  // with the stored dS the dQ kernel runs it in its tail
     bwd_dkrope_reduce_kernel<<<dim3((unsigned)((n_rope + 255) / 256)), dim3(256), 0, s>>>(prm);
   return launch_status("mla_prefill_bwd");

@@ -42,6 +42,7 @@ struct FwdParams {
   // q-tile whose keys span several segments leaves one partial per segment (O normalised
   // within the segment, fp32, and its log2 LSE) in ws_o / ws_lse for fwd_merge_kernel
   int S;
+  int single;  // one q-tile per workgroup, longest first (no key split), instead of mirrored pairs (TileGrid)
   float* ws_o;
   float* ws_lse;
   // RoPE folded into the Q load (rope_cos non-null): q_rope holds the unrotated rope slice and
@@ -95,7 +96,7 @@ constexpr float kFwdRescale = 8.0f;
 // the safe form; p <= 2^127 per key keeps every finite sum of the fast form exact up to it
 constexpr float kFwdSumLimit = 0x1p120f;
 
-// Maps the linear workgroup id to (b, h) and its pair of q-tiles.  A workgroup runs q-tiles
+// Maps the linear workgroup id to (b, h) and its pair of q-tiles (or, p.single, its one).  A workgroup runs q-tiles
 // n_qt - 1 - r and r of one (b, h) back to back: with causal masking the pair always
 // totals the same number of key tiles (balanced workgroups, no tail of short tiles) and
 // the second tile's first K/V tiles are loaded while the first one's output is stored.
@@ -104,6 +105,15 @@ constexpr float kFwdSumLimit = 0x1p120f;
 __device__ __forceinline__ void fwd_tile_coords(const FwdParams& p, int& b, int& h, int& qa, int& qb_, int& n_items) {
   const int n = gridDim.x;
   int id = blockIdx.x;
+  if (p.single) {  // (b, h) fastest: its tiles stay on one XCD when the (b, h) are a multiple of 8
+    const int n_bh = p.B * p.H;
+    const int t = id / n_bh, bh = id - t * n_bh;
+    qa = qb_ = p.n_qt - 1 - t;
+    n_items = 1;
+    b = bh / p.H;
+    h = bh - b * p.H;
+    return;
+  }
   if ((n & 7) == 0) id = (id & 7) * (n >> 3) + (id >> 3);
   const int n_pairs = (p.n_qt + 1) >> 1;
   const int bh = id / n_pairs;
@@ -903,7 +913,8 @@ static int launch_fwd(FwdParams prm, hipStream_t s, void* ws, size_t ws_bytes) {
   prm.S = 1;
   prm.ws_o = nullptr;
   prm.ws_lse = nullptr;
-  const int64_t n = (int64_t)prm.B * prm.H * ((prm.n_qt + 1) / 2);
+  prm.single = single_tiles_two_per_cu(TileGrid{(int64_t)prm.B * prm.H, prm.n_qt, prm.causal && prm.q_offset == 0});
+  const int64_t n = (int64_t)prm.B * prm.H * (prm.single ? prm.n_qt : (prm.n_qt + 1) / 2);
   MLA_CHECK(n < (1ll << 31), MLA_ERR_INVALID_ARG, "mla_prefill_fwd: grid too large");
   if (pt) prefill_fwd_kernel<DN, QB, true, false><<<dim3((unsigned)n), blk, 0, s>>>(prm);
   else prefill_fwd_kernel<DN, QB, false, false><<<dim3((unsigned)n), blk, 0, s>>>(prm);
