@@ -316,3 +316,22 @@ def test_decode_per_head_rope_keeps_a_heads_nan_to_it(ops):
     # each of at most 100 terms moves by 2^-8, which the parity bound of the oracle tests covers)
     check_close(ctx[0, same].double(), clean[0, same].double(), "other heads")
     assert ctx[0, 6].isnan().all()
+
+
+@pytest.mark.parametrize("B,H,L,DL,Hr", [
+    (24, 16, 1400, 256, 1),   # 10 splits: 240 workgroups
+    (40, 20, 500, 256, 1),    # 80 units of two head groups: 3 splits
+    (150, 16, 300, 384, 1),   # more units than half the CUs: one split
+    (300, 3, 40, 256, 3),     # more units than CUs
+    (24, 16, 1400, 128, 1),   # narrow latents share a CU: 11 splits
+])
+def test_decode_splits_stay_within_one_round(ops, B, H, L, DL, Hr):
+    print(f"case B={B} H={H} L={L} DL={DL} Hr={Hr}", flush=True)
+    q_lat, q_rope, c, kr = make(B, H, L, DL, Hr, seed=B + L)
+    scale = 1 / math.sqrt(192)
+    lens = [1 + (37 * b) % L for b in range(B)]
+    for sl in (None, lens):
+        ctx, lse = run(ops, q_lat, q_rope, c, kr, scale, sl)
+        rc, rl = oracle(q_lat, q_rope, c, kr, scale, None if sl is None else torch.tensor(sl))
+        check_close(ctx.double(), rc, "ctx")
+        torch.testing.assert_close(lse.double(), rl, rtol=0, atol=1e-3)
