@@ -147,3 +147,20 @@ def test_linear_double_backward_and_hooked_layers():
     h.remove()
     with torch.no_grad():
         assert not training.takes(lin, x)
+
+
+def test_batched_gradients_through_the_training_branch():
+    """A batch of gradients in one call (is_grads_batched) gives what one call for each gives: norm, attention branch and
+    o_proj, and a layer alone.  The two ways round at other places: three bf16 roundings of 2^-9, as many again inside."""
+    from transformer_amd import RMSNorm, training
+    m = _small()
+    norm = RMSNorm(256).cuda()
+    x = torch.randn(1, 70, 256, device="cuda").bfloat16().requires_grad_(True)
+    dy = torch.randn(3, 1, 70, 256, device="cuda").bfloat16()
+    leaves = [x, norm.weight] + list(m.parameters())
+    lin = m.o_proj
+    for y, at in ((m(norm(x))[0], leaves), (training.linear(x, lin.weight), [x, lin.weight])):
+        got = torch.autograd.grad(y, at, dy, is_grads_batched=True, retain_graph=True)
+        for i in range(3):
+            for a, b in zip(got, torch.autograd.grad(y, at, dy[i], retain_graph=True)):
+                assert (a[i].double() - b.double()).norm() <= 6 * 2.0 ** -9 * b.double().norm()

@@ -720,9 +720,8 @@ static int pick_splits(const mla_decode_args* a, int n_hg) {
   if (a->num_splits > 0) return (int)std::min<int64_t>(a->num_splits, std::max<int64_t>((a->L + 15) / 16, 1));
   const int64_t units = a->B * n_hg;
   // one workgroup per CU on 256 CUs (from d_latent 256 its registers leave no room for a second), and then never a few
-  // more: 11 splits
-  // of 24 sequences are 264 workgroups, a second round of 8.  Rounded up -> down (us, decode with W_UV, d_latent 512, 16
-  // heads): B = 24 over 4000 45.7 -> 35.9, B = 40 over 3000 53.4 -> 40.4, B = 48 over 4000 77.6 -> 55.6, B = 150 over 1000
+  // more: 11 splits of 24 sequences are 264 workgroups, a second round of 8.  Rounded up -> down (us, decode with W_UV,
+  // d_latent 512, 16 heads): B = 24 over 4000 45.7 -> 35.9, B = 40 over 3000 53.4 -> 40.4, B = 48 over 4000 77.6 -> 55.6, B = 150 over 1000
   // 71.5 -> 54.0 (one split); more rounds of smaller splits are slower at every batch measured (B = 48: 10 splits 63.7)
   int64_t s = a->d_latent >= 256 ? 256 / units : (256 + units - 1) / units;
   return (int)std::max<int64_t>(1, std::min<int64_t>(s, max_s));

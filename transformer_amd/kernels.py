@@ -1024,12 +1024,14 @@ def _(logits, targets, lse, g_vec, g_scale, v0):
 # ----------------------------------------------------------------- eager calls
 
 def _not_plain(args) -> bool:
-    """Tracing (torch.compile), a dispatch mode, a functorch transform, tensor subclasses, or tensors off the GPU."""
+    """Tracing (torch.compile), a dispatch mode, a functorch transform, tensor subclasses, batches of gradients
+    (is_grads_batched), or tensors off the GPU."""
     if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 \
             or torch._C._functorch.peek_interpreter_stack() is not None:
         return True
     for a in args:
-        if isinstance(a, Tensor) and ((type(a) is not Tensor and type(a) is not torch.nn.Parameter) or not a.is_cuda):
+        if isinstance(a, Tensor) and ((type(a) is not Tensor and type(a) is not torch.nn.Parameter) or not a.is_cuda
+                                      or torch._C._functorch.is_legacy_batchedtensor(a)):
             return True
     return False
 

@@ -8,8 +8,8 @@ reach fp32 weights as fp32: autocast's product rounds them to bf16 and casts the
 :306-315), as one Function whose backward writes each part of the down-projections' gradient where their product reads
 it.
 
-Callers take them only where nothing can tell the difference from ``nn.Linear`` (``takes``, ``takes_attention``); everything else (tracing,
-transforms, hooked or replaced submodules, other dtypes) keeps torch's own layers.
+Callers take them only where nothing can tell the difference from ``nn.Linear`` (``takes``, ``takes_attention``);
+everything else (tracing, transforms, hooked or replaced submodules, other dtypes) keeps torch's own layers.
 """
 from __future__ import annotations
 
@@ -79,6 +79,12 @@ def weight_grads(dy, x, weights, needed):
     return out
 
 
+def _by_operators(grad) -> bool:
+    """Whether a backward runs through operators that autograd and transforms see: it is itself differentiated, or
+    called with a batch of gradients (is_grads_batched) or under a dispatch mode."""
+    return torch.is_grad_enabled() or kernels._not_plain((grad,))
+
+
 class _Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, product, *weights):
@@ -91,7 +97,7 @@ class _Linear(torch.autograd.Function):
     def backward(ctx, dy):
         x, W = ctx.saved_tensors
         weights = ctx.weights
-        if torch.is_grad_enabled():  # the backward is itself differentiated: torch's operators on the inputs
+        if _by_operators(dy):  # torch's operators on the inputs
             W = torch.cat(weights, 0).to(x.dtype)
             dx = torch.matmul(dy, W)
             dW = torch.matmul(dy.reshape(-1, dy.size(-1)).t(), x.reshape(-1, x.size(-1)))
@@ -138,11 +144,11 @@ class _Attention(torch.autograd.Function):
         d, Wqb, Wkv, q, q_rot, kv, k_rope, o, lse, cos, sin = ctx.saved_tensors
         H, dn, dv, hr, ql, dl = ctx.layout
         B, T, n = d.shape
-        if torch.is_grad_enabled():  # the backward is itself differentiated: through the operators
+        if _by_operators(do):
             inputs = [t for t, need in zip((d, *ctx.weights), ctx.needs_input_grad) if need]
             with torch.enable_grad():
                 out = _attention_by_operators(d, *ctx.weights, cos, sin, ctx.layout, ctx.scale)
-            got = iter(torch.autograd.grad(out, inputs, do, create_graph=True))
+            got = iter(torch.autograd.grad(out, inputs, do, create_graph=torch.is_grad_enabled()))
             return tuple(next(got) if need else None for need in ctx.needs_input_grad[:4]) + (None,) * 4
         d2 = d.reshape(B * T, n)
         dd = torch.empty(B * T, n, dtype=d.dtype, device=d.device)
