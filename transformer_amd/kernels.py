@@ -141,7 +141,7 @@ def _rope_setup(ctx, inputs, output):
 def _rope_backward(ctx, grad):
     cos, sin = ctx.saved_tensors
     # R is orthogonal: the gradient is the rotation by the opposite angle
-    return eager.rope(grad, cos, sin, ctx.pos_offset, not ctx.inverse), None, None, None, None
+    return _ops_for(grad).rope(grad, cos, sin, ctx.pos_offset, not ctx.inverse), None, None, None, None
 
 
 _register_autograd(rope, "rope", _rope_setup, _rope_backward)
@@ -433,7 +433,7 @@ def _prefill_setup(ctx, inputs, output):
 
 def _prefill_backward(ctx, do, dlse):
     q_nope, q_rope, k_nope, k_rope, v, o, lse = ctx.saved_tensors
-    grads = eager.prefill_bwd(do, q_nope, q_rope, k_nope, k_rope, v, o, lse, ctx.scale, ctx.causal, ctx.q_offset)
+    grads = _ops_for(do).prefill_bwd(do, q_nope, q_rope, k_nope, k_rope, v, o, lse, ctx.scale, ctx.causal, ctx.q_offset)
     return (*grads, None, None, None)
 
 
@@ -453,7 +453,7 @@ def _prefill_rope_backward(ctx, do, dlse, dqrot):
     if not ctx.saved_rotated:
         raise RuntimeError("prefill_fwd_rope: the backward needs save_rotated=True in the forward")
     q_nope, q_rot, k_nope, k_rope, v, o, lse, cos, sin = ctx.saved_tensors
-    grads = eager.prefill_bwd(do, q_nope, q_rot, k_nope, k_rope, v, o, lse, ctx.scale, ctx.causal, ctx.q_offset, cos,
+    grads = _ops_for(do).prefill_bwd(do, q_nope, q_rot, k_nope, k_rope, v, o, lse, ctx.scale, ctx.causal, ctx.q_offset, cos,
                               sin, ctx.q_pos_offset)
     return (*grads, None, None, None, None, None, None, None)
 
@@ -921,7 +921,7 @@ def _rms_setup(ctx, inputs, output):
 
 def _rms_backward(ctx, dy, dinv):
     x, weight, inv = ctx.saved_tensors
-    dx, dw = eager.rmsnorm_bwd(dy, x, weight, inv)
+    dx, dw = _ops_for(dy).rmsnorm_bwd(dy, x, weight, inv)
     return dx, dw.to(weight.dtype), None, None
 
 
@@ -1024,16 +1024,24 @@ def _(logits, targets, lse, g_vec, g_scale, v0):
 # ----------------------------------------------------------------- eager calls
 
 def _not_plain(args) -> bool:
-    """Tracing (torch.compile), a dispatch mode, a functorch transform, tensor subclasses, batches of gradients
-    (is_grads_batched), or tensors off the GPU."""
+    """Tracing (torch.compile), a dispatch mode, a functorch transform, tensor subclasses, or tensors off the GPU."""
     if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 \
             or torch._C._functorch.peek_interpreter_stack() is not None:
         return True
     for a in args:
-        if isinstance(a, Tensor) and ((type(a) is not Tensor and type(a) is not torch.nn.Parameter) or not a.is_cuda
-                                      or torch._C._functorch.is_legacy_batchedtensor(a)):
+        if isinstance(a, Tensor) and ((type(a) is not Tensor and type(a) is not torch.nn.Parameter) or not a.is_cuda):
             return True
     return False
+
+
+def batched_grad(grad: Tensor) -> bool:
+    """Whether a backward was handed a batch of gradients (is_grads_batched): tensors without storage."""
+    return torch._C._functorch.is_legacy_batchedtensor(grad)
+
+
+def _ops_for(grad: Tensor):
+    """The operators that a backward formula runs on ``grad``."""
+    return torch.ops.mla_mi355x if batched_grad(grad) else eager
 
 
 def _needs_grad(args) -> bool:

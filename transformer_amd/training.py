@@ -82,7 +82,7 @@ def weight_grads(dy, x, weights, needed):
 def _by_operators(grad) -> bool:
     """Whether a backward runs through operators that autograd and transforms see: it is itself differentiated, or
     called with a batch of gradients (is_grads_batched) or under a dispatch mode."""
-    return torch.is_grad_enabled() or kernels._not_plain((grad,))
+    return torch.is_grad_enabled() or kernels.batched_grad(grad) or kernels._not_plain((grad,))
 
 
 class _Linear(torch.autograd.Function):
