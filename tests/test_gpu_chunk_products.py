@@ -1,0 +1,38 @@
+"""The products around a chunk over a cache, at sizes off the tiles."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("weights", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dims", ["baseline", "default"])
+@pytest.mark.parametrize("B,T,L", [(1, 2, 5), (3, 13, 70), (2, 129, 33), (2, 33, 0)])
+def test_chunk_equals_the_same_layer_with_hooks(B, T, L, dims, weights):
+    """A hook on k_up keeps it a product of its own; the absorbed form has none to keep, so it is also compared with the
+    form over per-head K and V.  bf16 operands, stored K, V and outputs: a few roundings of 2^-9 each way."""
+    from contextlib import nullcontext
+    from transformer_amd import MLA, ModelArgs, mla
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs.mla_baseline() if dims == "baseline" else ModelArgs())  # bf16 RoPE tables
+        m = m.to(weights) if weights == torch.bfloat16 else m
+        x = torch.randn(B, T, m.d_model).to(weights)
+        cache = None
+        if L:
+            cache = {"latent": torch.randn(B, L, m.d_latent).bfloat16(),
+                     "k_rope": torch.randn(B, m.n_k_rope_heads, L, 64).bfloat16(), "seq_len": L}
+    amp = nullcontext() if weights == torch.bfloat16 else torch.autocast("cuda", torch.bfloat16)
+    with torch.no_grad(), amp:
+        y = m(x, cache, True)[0]
+        h = m.k_up.register_forward_hook(lambda *a: None)
+        old, mla.ABSORBED_PREFILL = mla.ABSORBED_PREFILL, False
+        try:
+            want = m(x, cache, True)[0]
+        finally:
+            mla.ABSORBED_PREFILL = old
+            h.remove()
+        assert y.shape == want.shape and y.dtype == want.dtype
+        assert (y.double() - want.double()).norm() <= 8 * 2.0 ** -9 * want.double().norm()
+        m.v_up.weight.mul_(2)  # the kept weights follow
+        assert not torch.equal(m(x, cache, True)[0], y)

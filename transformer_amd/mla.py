@@ -192,7 +192,7 @@ class MLA(nn.Module):
         """A derived weight (``make()``, cast to ``dtype``) kept while the parameters it reads
         are unchanged (same storage and version counter); autograd off only."""
         params = [self.q_down.weight, self.qk_rope.weight, self.kv_down.weight] if name == "down" else \
-            [getattr(self, name.split(":")[0]).weight]
+            [self.k_up.weight, self.v_up.weight] if name == "kv_up" else [getattr(self, name.split(":")[0]).weight]
         key = tuple((w.data_ptr(), w._version) for w in params) + (dtype,)
         cache = self.__dict__.setdefault("_derived", {})
         hit = cache.get(name)
@@ -339,6 +339,13 @@ class MLA(nn.Module):
         if torch.is_grad_enabled() and x.requires_grad:  # frozen weights, the input's gradient
             return training.linear(x.to(W.dtype), W, product=_down_product)
         return _linear_split_cols(x.to(W.dtype), W)
+
+    def _kv_up_as_one(self, kv_latent):
+        """Whether ``k_up`` and ``v_up`` over a cache may be one bf16 product: autograd off, both plain layers in bf16
+        arithmetic, eager."""
+        return (not torch.is_grad_enabled() and kv_latent.dtype == torch.bfloat16
+                and all(training._bf16_arithmetic(self._modules[n], kv_latent) for n in ("k_up", "v_up"))
+                and training.plain_call(kv_latent))
 
     def _proj(self, name, x):
         """``self.<name>(x)``, with the weight gradient on this package's kernel where that is all the layer does."""
@@ -489,17 +496,27 @@ class MLA(nn.Module):
             # latent rows on prefill_cached (query t at position pos_offset + t)
             DL = self.d_latent
             Wk = self._cached_weight("k_up", lambda: self.k_up.weight.view(H, dn, DL), torch.bfloat16)
-            qn = b(q_nope).permute(2, 0, 1, 3).reshape(H, B * T, dn)
-            q_lat = torch.bmm(qn, Wk).view(H, B, T, DL).permute(1, 2, 0, 3)  # [B,T,H,DL] view
+            # q_nope stays where it is (a head's rows H dn apart) and the last product writes where o_proj reads: no copies
+            q_lat = torch.bmm(b(q_nope).reshape(B * T, H, dn).transpose(0, 1), Wk)  # [H,B*T,DL]
+            q_lat = q_lat.view(H, B, T, DL).permute(1, 2, 0, 3)  # [B,T,H,DL] view
             ctx, _ = ops.prefill_cached(q_lat, b(q_rope), b(kv_latent), b(k_pos), pos_offset, self.scale, True)
             Wvt = self._cached_weight("v_up:t", lambda: self.v_up.weight.view(H, dv, DL).transpose(1, 2),
                                       torch.bfloat16)  # [H, DL, dv]
-            out = torch.bmm(ctx.permute(2, 0, 1, 3).reshape(H, B * T, DL), Wvt)  # [H, B*T, dv]
-            out = out.view(H, B, T, dv).permute(1, 2, 0, 3).reshape(B, T, H * dv).to(cdt)
+            out = torch.empty(B * T, H, dv, dtype=torch.bfloat16, device=x.device)
+            torch.bmm(ctx.permute(2, 0, 1, 3).reshape(H, B * T, DL), Wvt, out=out.transpose(0, 1))
+            out = out.view(B, T, H * dv).to(cdt)
         else:
             # T > 1 with the bottom-right causal mask of :273-281 (q_offset = pos_offset)
-            k_nope = self.k_up(kv_latent).view(B, kv_len, H, dn)
-            v = self.v_up(kv_latent).view(B, kv_len, H, dv)
+            if self._kv_up_as_one(kv_latent):
+                # K and V as the column views of one product over weights kept in bf16: the latent rows are read once, and
+                # the launches bound a chunk (B = 4, T = 75 over 2500, default dims, fp32 weights: 278 -> 257 us)
+                W = self._cached_weight("kv_up", lambda: torch.cat([self.k_up.weight, self.v_up.weight], 0),
+                                        torch.bfloat16)
+                kv = torch.mm(kv_latent.reshape(B * kv_len, self.d_latent), W.t())
+                k_nope, v = training._kv_views(kv, B, kv_len, H, dn, dv)
+            else:
+                k_nope = self.k_up(kv_latent).view(B, kv_len, H, dn)
+                v = self.v_up(kv_latent).view(B, kv_len, H, dv)
             o, _ = ops.prefill_fwd(b(q_nope), b(q_rope), b(k_nope), b(k_pos.transpose(1, 2)), b(v), self.scale,
                                    True, pos_offset)
             out = o.reshape(B, T, H * dv).to(cdt)
