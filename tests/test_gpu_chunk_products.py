@@ -36,3 +36,29 @@ def test_chunk_equals_the_same_layer_with_hooks(B, T, L, dims, weights):
         assert (y.double() - want.double()).norm() <= 8 * 2.0 ** -9 * want.double().norm()
         m.v_up.weight.mul_(2)  # the kept weights follow
         assert not torch.equal(m(x, cache, True)[0], y)
+
+
+def test_recorded_chunk_follows_its_weights():
+    """A recorded chunk reads k_up and v_up themselves: replays after an update give the updated layer's outputs."""
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(4)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs()).to(torch.bfloat16)
+        x = torch.randn(1, 9, m.d_model).bfloat16()
+        cache = {"latent": torch.randn(1, 40, m.d_latent).bfloat16(),
+                 "k_rope": torch.randn(1, m.n_k_rope_heads, 40, 64).bfloat16(), "seq_len": 40}
+    with torch.no_grad():
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            for _ in range(2):
+                m(x, dict(cache), True)
+        torch.cuda.current_stream().wait_stream(s)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = m(x, dict(cache), True)[0]
+        for _ in range(3):
+            graph.replay()
+            want = m(x, dict(cache), True)[0]
+            assert (y.double() - want.double()).norm() <= 4 * 2.0 ** -9 * want.double().norm()
+            m.v_up.weight.mul_(0.5)

@@ -342,8 +342,10 @@ class MLA(nn.Module):
 
     def _kv_up_as_one(self, kv_latent):
         """Whether ``k_up`` and ``v_up`` over a cache may be one bf16 product: autograd off, both plain layers in bf16
-        arithmetic, eager."""
+        arithmetic, eager.  Not in a capture: a recorded call reads the weights themselves, so a replay sees them as
+        they then are."""
         return (not torch.is_grad_enabled() and kv_latent.dtype == torch.bfloat16
+                and not torch.cuda.is_current_stream_capturing()
                 and all(training._bf16_arithmetic(self._modules[n], kv_latent) for n in ("k_up", "v_up"))
                 and training.plain_call(kv_latent))
 
