@@ -335,7 +335,7 @@ class MLA(nn.Module):
             self._down_key = key
         W = self._down_w
         if not split:
-            return torch.nn.functional.linear(x, W)
+            return training.on_rows(torch.nn.functional.linear, x, W).view(*x.shape[:-1], W.size(0))
         if torch.is_grad_enabled() and x.requires_grad:  # frozen weights, the input's gradient
             return training.linear(x.to(W.dtype), W, product=_down_product)
         return _linear_split_cols(x.to(W.dtype), W)
@@ -517,8 +517,10 @@ class MLA(nn.Module):
                 kv = torch.mm(kv_latent.reshape(B * kv_len, self.d_latent), W.t())
                 k_nope, v = training._kv_views(kv, B, kv_len, H, dn, dv)
             else:
-                k_nope = self.k_up(kv_latent).view(B, kv_len, H, dn)
-                v = self.v_up(kv_latent).view(B, kv_len, H, dv)
+                # evenly spaced rows: the cache's are not, and frozen weights would make a batched product (on_rows)
+                lat = kv_latent.reshape(B * kv_len, self.d_latent).view(B, kv_len, self.d_latent)
+                k_nope = self.k_up(lat).view(B, kv_len, H, dn)
+                v = self.v_up(lat).view(B, kv_len, H, dv)
             o, _ = ops.prefill_fwd(b(q_nope), b(q_rope), b(k_nope), b(k_pos.transpose(1, 2)), b(v), self.scale,
                                    True, pos_offset)
             out = o.reshape(B, T, H * dv).to(cdt)

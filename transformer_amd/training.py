@@ -85,26 +85,35 @@ def _by_operators(grad) -> bool:
     return torch.is_grad_enabled() or kernels.batched_grad(grad) or kernels._not_plain((grad,))
 
 
+def on_rows(product, x, W):
+    """``product(x, W) [rows, N]`` over x's rows as one matrix.  torch's own product of a batch whose rows are not evenly
+    spaced (a slice of longer sequences, a transpose) with a weight that needs no gradient is a batched one over the
+    expanded transpose of the weight: slow, and bf16 batched products with a transposed right operand have faulted on
+    this GPU."""
+    return product(x.reshape(-1, x.size(-1)), W)
+
+
 class _Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, product, *weights):
         W = cat_weights(weights, x.dtype)
         ctx.save_for_backward(x, W)
         ctx.weights = weights
-        return product(x, W)
+        # (no view, as torch's own output is none: callers may change it in place)
+        return torch.ops.aten._unsafe_view.default(on_rows(product, x, W), (*x.shape[:-1], W.size(0)))
 
     @staticmethod
     def backward(ctx, dy):
         x, W = ctx.saved_tensors
         weights = ctx.weights
+        dy2, x2 = dy.reshape(-1, dy.size(-1)), x.reshape(-1, x.size(-1))
         if _by_operators(dy):  # torch's operators on the inputs
             W = torch.cat(weights, 0).to(x.dtype)
-            dx = torch.matmul(dy, W)
-            dW = torch.matmul(dy.reshape(-1, dy.size(-1)).t(), x.reshape(-1, x.size(-1)))
+            dx = torch.matmul(dy2, W).view(x.shape)
+            dW = torch.matmul(dy2.t(), x2)
             return (dx, None) + tuple(g.to(w.dtype) for g, w in zip(dW.split([w.size(0) for w in weights]), weights))
-        dx = torch.matmul(dy, W) if ctx.needs_input_grad[0] else None
-        grads = weight_grads(dy.reshape(-1, dy.size(-1)), x.reshape(-1, x.size(-1)), weights, ctx.needs_input_grad[2:])
-        return (dx, None, *grads)
+        dx = torch.matmul(dy2, W).view(x.shape) if ctx.needs_input_grad[0] else None
+        return (dx, None, *weight_grads(dy2, x2, weights, ctx.needs_input_grad[2:]))
 
 
 def linear(x: torch.Tensor, *weights, product=torch.nn.functional.linear) -> torch.Tensor:
