@@ -62,3 +62,57 @@ def test_recorded_chunk_follows_its_weights():
             want = m(x, dict(cache), True)[0]
             assert (y.double() - want.double()).norm() <= 4 * 2.0 ** -9 * want.double().norm()
             m.v_up.weight.mul_(0.5)
+
+
+@pytest.mark.parametrize("dims", ["baseline", "default"])
+def test_recorded_few_row_chunk_follows_fp32_projections(dims):
+    """fp32 weights under autocast, at most 64 rows: replays after an update of q_up, o_proj (and, where they are layers,
+    k_up and v_up) give the updated layer's outputs.  Both round bf16 weights and results: a few times 2^-9."""
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(6)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs.mla_baseline() if dims == "baseline" else ModelArgs())
+        x = torch.randn(2, 9, m.d_model)
+        cache = {"latent": torch.randn(2, 40, m.d_latent).bfloat16(),
+                 "k_rope": torch.randn(2, m.n_k_rope_heads, 40, 64).bfloat16(), "seq_len": 40}
+    with torch.no_grad(), torch.autocast("cuda", torch.bfloat16, cache_enabled=False):
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            for _ in range(2):
+                m(x, dict(cache), True)
+        torch.cuda.current_stream().wait_stream(s)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = m(x, dict(cache), True)[0]
+        for i in range(4):
+            graph.replay()
+            want = m(x, dict(cache), True)[0]
+            assert (y.double() - want.double()).norm() <= 4 * 2.0 ** -9 * want.double().norm(), i
+            for name in ("q_up", "o_proj") + (("k_up", "v_up") if dims == "default" else ()):
+                m._modules[name].weight.mul_(1.25 if i % 2 else 0.5)
+
+
+@pytest.mark.parametrize("dims", ["baseline", "default"])
+@pytest.mark.parametrize("B,T,L", [(1, 1, 30), (4, 10, 0), (2, 9, 40)])
+def test_few_row_calls_run_hooked_projections(B, T, L, dims):
+    """A hook on q_up that doubles its output does what doubling its weight does (exact in bf16), and one on o_proj runs."""
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(7)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs.mla_baseline() if dims == "baseline" else ModelArgs()).to(torch.bfloat16)
+        x = torch.randn(B, T, m.d_model).bfloat16()
+        cache = None
+        if L:
+            cache = {"latent": torch.randn(B, L, m.d_latent).bfloat16(),
+                     "k_rope": torch.randn(B, m.n_k_rope_heads, L, 64).bfloat16(), "seq_len": L}
+    seen = []
+    with torch.no_grad():
+        hook = m.o_proj.register_forward_hook(lambda mod, a, y: seen.append(1))
+        h = m.q_up.register_forward_hook(lambda mod, a, y: y * 2)
+        y = m(x, cache, True)[0]
+        h.remove()
+        m.q_up.weight.mul_(2)
+        want = m(x, cache, True)[0]
+        hook.remove()
+    assert len(seen) == 2 and torch.equal(y, want)

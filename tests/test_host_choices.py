@@ -203,3 +203,70 @@ def test_rows_path_takes_the_projections_where_only_the_absorption_does_not_fit(
     with torch.no_grad():
         assert m._rows_proj_ok() and not m._rows_dims_ok() and m._rows_path(x)
         assert not m._rows_path(torch.zeros(65, 1, m.d_model, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("baseline", [True, False])
+@pytest.mark.parametrize("layer", ["q_up", "o_proj"])
+def test_rows_path_calls_layers_that_are_more_than_a_product(layer, baseline):
+    # a hook, a wrapper that passes the weight on (an adapter), a parametrization (a fresh weight on each access), a layer
+    # of another kind: the few-row products read weights, so they give way to the layers' own calls
+    from transformer_amd import MLA, ModelArgs
+    import torch.nn as nn
+
+    class Adapter(nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        @property
+        def weight(self):
+            return self.inner.weight
+
+        def forward(self, x):
+            return self.inner(x) * 2
+
+    def make():
+        m = MLA(ModelArgs.mla_baseline(max_seq_len=64) if baseline else ModelArgs(max_seq_len=64)).to(torch.bfloat16)
+        return m, m._modules[layer]
+
+    def hooked(m, lin):
+        lin.register_forward_hook(lambda *a: None)
+
+    def wrapped(m, lin):
+        m._modules[layer] = Adapter(lin)
+
+    def several(m, lin):
+        m._modules[layer] = nn.Sequential(lin)
+
+    def parametrized(m, lin):
+        nn.utils.parametrize.register_parametrization(lin, "weight", nn.Identity())
+
+    with torch.no_grad():
+        for change in (None, hooked, wrapped, several, parametrized):
+            m, lin = make()
+            x = torch.zeros(40, 1, m.d_model, dtype=torch.bfloat16)
+            if change:
+                change(m, lin)
+            assert m._rows_path(x) == (change is None), change
+
+
+def test_rows_path_keeps_no_copies_of_fp32_weights_where_the_layers_ran(monkeypatch):
+    # fp32 weights under bf16 autocast: the reference's default dims keep q_up and o_proj as layers, and no layout reads a
+    # kept copy in a capture; bf16 weights are read as they are
+    from transformer_amd import MLA, ModelArgs
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    amp = [True]
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *a: amp[0])  # (no GPU: torch turns autocast off)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda *a: torch.bfloat16)
+    for baseline in (True, False):
+        m = MLA(ModelArgs.mla_baseline(max_seq_len=64) if baseline else ModelArgs(max_seq_len=64))
+        x = torch.zeros(2, 1, m.d_model)
+        with torch.no_grad():
+            for weights in (torch.float32, torch.bfloat16):
+                m = m.to(weights)
+                amp[0] = True
+                for capturing[0] in (False, True):
+                    assert m._rows_path(x) == (weights == torch.bfloat16 or (baseline and not capturing[0]))
+            amp[0] = False
+            assert m._rows_path(x) == baseline  # no autocast, fp32 x, bf16 weights: torch's layer refuses it at the default dims

@@ -297,13 +297,26 @@ class MLA(nn.Module):
             (self.d_model, n_down), (self.q_up.weight.size(1), H * dn), (H * dv, self.d_model)))
 
     def _rows_path(self, x):
-        """Few-row bf16 products (the decode step): autograd off, at most ROWS_FAST_M rows, and
-        bf16 arithmetic (bf16 weights, or bf16 autocast)."""
-        if torch.is_grad_enabled() or x.size(0) * x.size(1) > kernels.ROWS_FAST_M or not self._rows_proj_ok():
+        """Few-row bf16 products (the decode step): autograd off, at most ROWS_FAST_M rows, bf16 arithmetic (bf16
+        weights, or bf16 autocast), and ``q_up`` and ``o_proj`` plain layers: a hooked, wrapped or parametrized one is
+        called.  fp32 weights would be read from kept bf16 copies: not in a capture, whose replays would no longer
+        follow the weights, and only where the whole step fits linear_rows."""
+        if torch.is_grad_enabled() or x.size(0) * x.size(1) > kernels.ROWS_FAST_M or not self._plain_projections() \
+                or not self._rows_proj_ok():
             return False
-        if torch.is_autocast_enabled("cuda"):
-            return torch.get_autocast_dtype("cuda") == torch.bfloat16
-        return self.o_proj.weight.dtype == torch.bfloat16
+        amp = torch.is_autocast_enabled("cuda")
+        wq, wo = self._modules["q_up"].weight.dtype, self._modules["o_proj"].weight.dtype
+        if (torch.get_autocast_dtype("cuda") if amp else wo) != torch.bfloat16:
+            return False
+        whole = kernels.rows_fit(self.content_dim, self.d_latent)
+        if wq == torch.bfloat16 and wo == torch.bfloat16:
+            return whole or amp or x.dtype == torch.bfloat16
+        return whole and not torch.cuda.is_current_stream_capturing()
+
+    def _plain_projections(self):
+        """Whether calling ``q_up`` and ``o_proj`` is no more than a product with their weights."""
+        mods = self._modules
+        return training.plain_linear(mods["q_up"]) and training.plain_linear(mods["o_proj"])
 
     def _down_proj(self, x):
         """The column views of :meth:`_down_all`: ``q_down(x)``, ``qk_rope(x)`` and ``kv_down(x)``."""

@@ -27,9 +27,12 @@ def plain_call(*tensors) -> bool:
 
 def plain_linear(m: nn.Module) -> bool:
     """Whether calling ``m`` is no more than ``x @ m.weight^T``: an nn.Linear without bias, hooks or an override."""
-    return (type(m) is nn.Linear and m.bias is None and type(m._parameters.get("weight")) is nn.Parameter
-            and "forward" not in m.__dict__
-            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+    if type(m) is not nn.Linear:
+        return False
+    d = m.__dict__  # (a decode step asks on every call: attribute lookups on a module take twice as long)
+    p = d["_parameters"]
+    return (type(p.get("weight")) is nn.Parameter and p.get("bias") is None and "forward" not in d
+            and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"])
             and not _nn_module._has_any_global_hook())
 
 
