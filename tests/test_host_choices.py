@@ -207,11 +207,12 @@ def test_rows_path_takes_the_projections_where_only_the_absorption_does_not_fit(
 
 @pytest.mark.parametrize("baseline", [True, False])
 @pytest.mark.parametrize("layer", ["q_up", "o_proj"])
-def test_rows_path_calls_layers_that_are_more_than_a_product(layer, baseline):
+def test_rows_path_calls_layers_that_are_more_than_a_product(layer, baseline, monkeypatch):
     # a hook, a wrapper that passes the weight on (an adapter), a parametrization (a fresh weight on each access), a layer
     # of another kind: the few-row products read weights, so they give way to the layers' own calls
     from transformer_amd import MLA, ModelArgs
     import torch.nn as nn
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)  # (asks a GPU)
 
     class Adapter(nn.Module):
         def __init__(self, inner):
@@ -248,6 +249,7 @@ def test_rows_path_calls_layers_that_are_more_than_a_product(layer, baseline):
             if change:
                 change(m, lin)
             assert m._rows_path(x) == (change is None), change
+            assert m._auto_graph_ok(x) == (change is None), change
 
 
 def test_rows_path_keeps_no_copies_of_fp32_weights_where_the_layers_ran(monkeypatch):

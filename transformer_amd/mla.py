@@ -206,11 +206,12 @@ class MLA(nn.Module):
         """The one-token cached step may replay a recorded graph: autograd off; with autocast off,
         bf16 weights and a bf16 input; under bf16 autocast, bf16 or fp32 weights and a bf16 or fp32
         input (fp32 weights under bf16 autocast is how the reference's generation loop runs,
-        CLI.py:294); not inside a graph capture or torch.compile, and the module has not given up
-        recording.  The recording keeps its cache in bf16, which is the reference's cache dtype in
+        CLI.py:294); q_up and o_proj plain layers (the recording reads their weights: a hooked, wrapped or
+        parametrized one is called eagerly); not inside a graph capture or torch.compile, and the module has
+        not given up recording.  The recording keeps its cache in bf16, which is the reference's cache dtype in
         those cases; an fp32 module outside autocast takes the eager kernels, whose cache stays
         fp32 as the reference's does (transformer.py:215-218, :241-244)."""
-        if not AUTO_GRAPH or torch.is_grad_enabled():
+        if not AUTO_GRAPH or torch.is_grad_enabled() or not self._plain_projections():
             return False
         wdt, amp = self._step_weights()[-1].dtype, torch.is_autocast_enabled("cuda")
         if amp:
