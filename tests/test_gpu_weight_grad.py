@@ -164,3 +164,30 @@ def test_batched_gradients_through_the_training_branch():
         for i in range(3):
             for a, b in zip(got, torch.autograd.grad(y, at, dy[i], retain_graph=True)):
                 assert (a[i].double() - b.double()).norm() <= 6 * 2.0 ** -9 * b.double().norm()
+
+
+@pytest.mark.parametrize("weights", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B", [1, 2])
+def test_expanded_gradients_and_overlapping_inputs(B, weights):
+    """Gradients of sums (stride 0 over tokens, columns or both) and inputs whose rows repeat or overlap give what the
+    same values as plain tensors give."""
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(8)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=128)).to(weights)
+    base = torch.randn(256 * 80, device="cuda").bfloat16()
+    col = torch.randn(256, device="cuda").bfloat16()
+    inputs = [base.as_strided((B, 37, 256), (128, 256, 1)), base.as_strided((B, 37, 256), (8, 128, 1)),
+              base[:256].expand(B, 37, 256)]
+
+    def grads(x, reduce):
+        with torch.autocast("cuda", torch.bfloat16, enabled=weights == torch.float32):
+            y = m(x)[0]
+        return torch.autograd.grad(reduce(y), list(m.parameters()))
+
+    for x in inputs:
+        for reduce in (lambda y: y.float().sum(), lambda y: (y.sum((0, 1)) * col).sum(), lambda y: (y.sum(1) * col).sum(),
+                       lambda y: y.sum()):
+            got = grads(x, reduce)
+            want = grads(x.clone(memory_format=torch.contiguous_format), reduce)
+            assert all(torch.equal(a, b) for a, b in zip(got, want))

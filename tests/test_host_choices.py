@@ -272,3 +272,18 @@ def test_rows_path_keeps_no_copies_of_fp32_weights_where_the_layers_ran(monkeypa
                     assert m._rows_path(x) == (weights == torch.bfloat16 or (baseline and not capturing[0]))
             amp[0] = False
             assert m._rows_path(x) == baseline  # no autocast, fp32 x, bf16 weights: torch's layer refuses it at the default dims
+
+
+def test_weight_gradient_rows_do_not_overlap():
+    # strides that torch's products take and mla_weight_grad refuses (rows that overlap or repeat, an inner stride, odd
+    # strides) are copied, before the limits are asked; others are passed as they are
+    from transformer_amd import kernels
+    rows = kernels.weight_grad_rows
+    b = torch.randn(16, 64, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    flat = b.view(-1)
+    for t in (b[:1, :1].expand(9, 16), b[0, :16].expand(9, 16), b[:, :1].expand(16, 16), b.t(), b[:, ::2], b[:, 1:17],
+              flat.as_strided((9, 16), (8, 1)), flat.as_strided((9, 16), (20, 1))):
+        r = rows(t)
+        assert torch.equal(r, t) and r.stride(1) == 1 and r.stride(0) >= r.size(1) and r.stride(0) % 8 == 0
+    for t in (b, b[:, 8:40], b[:1, :16]):
+        assert rows(t) is t

@@ -930,6 +930,13 @@ _register_autograd(rmsnorm, "rmsnorm", _rms_setup, _rms_backward)
 
 # ----------------------------------------------------------------- weight gradient
 
+def weight_grad_rows(t: Tensor) -> Tensor:
+    """``t [M, N]`` as the kernel takes it: unit inner stride, whole 16-byte runs, rows that do not overlap.  A sum's
+    gradient (expanded, stride 0), an expanded input or windows of one buffer are copied."""
+    t = _aligned4(t, 8)
+    return t.contiguous() if t.size(0) > 1 and t.stride(0) < t.size(1) else t
+
+
 def weight_grad_fits(M: int, N: int, K: int, dy_stride: int, x_stride: int) -> bool:
     """Whether a [M, N]^T x [M, K] product is within weight_grad's limits (see mla_mi355x.h)."""
     return 0 < M < 1 << 24 and 0 < N < 1 << 20 and 0 < K < 1 << 20 and N % 8 == 0 and K % 8 == 0 \
@@ -945,7 +952,7 @@ def weight_grad(dy: Tensor, x: Tensor, out_fp32: bool = False) -> Tensor:
     _bf16(op, dy=dy, x=x)
     if dy.dim() != 2 or x.dim() != 2 or dy.size(0) != x.size(0):
         raise ValueError(f"{op}: expected dy [M, N] and x [M, K]; got {tuple(dy.shape)}, {tuple(x.shape)}")
-    dy, x = _aligned4(dy, 8), _aligned4(x, 8)
+    dy, x = weight_grad_rows(dy), weight_grad_rows(x)
     (M, N), K = dy.shape, x.size(1)
     sy, sx = (dy.stride(0), x.stride(0)) if M > 1 else (N, K)
     if not weight_grad_fits(M, N, K, sy, sx):

@@ -70,10 +70,12 @@ def weight_grads(dy, x, weights, needed):
     if not any(needed):
         return [None] * len(weights)
     f32 = all(w.dtype == torch.float32 for w in weights)
-    sy, sx = dy.stride(0), x.stride(0)
-    if dy.dtype == torch.bfloat16 and kernels.weight_grad_fits(dy.size(0), dy.size(1), x.size(1), sy, sx):
-        dW = kernels.weight_grad(dy, x, f32)
-    else:
+    dW = None
+    if dy.dtype == torch.bfloat16:
+        dyr, xr = kernels.weight_grad_rows(dy), kernels.weight_grad_rows(x)
+        if kernels.weight_grad_fits(*dy.shape, x.size(1), dyr.stride(0), xr.stride(0)):
+            dW = kernels.weight_grad(dyr, xr, f32)
+    if dW is None:
         dW = torch.matmul(dy.t(), x)
     out, r = [], 0
     for w, need in zip(weights, needed):
