@@ -287,3 +287,16 @@ def test_weight_gradient_rows_do_not_overlap():
         assert torch.equal(r, t) and r.stride(1) == 1 and r.stride(0) >= r.size(1) and r.stride(0) % 8 == 0
     for t in (b, b[:, 8:40], b[:1, :16]):
         assert rows(t) is t
+
+
+def test_contiguous_rows_off_the_alignment_are_copied():
+    # a slice of a flat buffer at an odd offset is contiguous: contiguous() returns it as it is, and every entry point
+    # refuses an operand that is not 16-byte aligned
+    from transformer_amd import kernels
+    flat = torch.arange(200, dtype=torch.float32).to(torch.bfloat16)
+    for t in (flat[1:129].view(8, 16), flat[3:131].view(2, 4, 16)):
+        a = kernels._aligned4(t, 8)
+        assert a.data_ptr() % 16 == 0 and a.is_contiguous() and torch.equal(a, t)
+    assert kernels.weight_grad_rows(flat[1:129].view(8, 16)).data_ptr() % 16 == 0
+    whole = flat[8:136].view(8, 16)
+    assert kernels._aligned4(whole, 8) is whole

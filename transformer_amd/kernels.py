@@ -69,7 +69,10 @@ def _aligned4(t: Tensor, vec_elems: int) -> Tensor:
     base and strides that are multiples of ``vec_elems`` elements."""
     ok = (t.stride(-1) == 1 or t.size(-1) == 1) and t.data_ptr() % 16 == 0 and all(
         s % vec_elems == 0 for s, n in zip(t.stride()[:-1], t.shape[:-1]) if n > 1)
-    return t if ok else t.contiguous()
+    if ok:
+        return t
+    c = t.contiguous()
+    return c if c.data_ptr() % 16 == 0 else c.clone()  # (contiguous, but off the alignment)
 
 
 def _st4(t: Tensor, zero_head: bool = False) -> Strides:
