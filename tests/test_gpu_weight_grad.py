@@ -191,3 +191,21 @@ def test_expanded_gradients_and_overlapping_inputs(B, weights):
             got = grads(x, reduce)
             want = grads(x.clone(memory_format=torch.contiguous_format), reduce)
             assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("name", ["q_up", "k_up", "v_up", "o_proj"])
+def test_replaced_layers_train_through_their_own_call(name):
+    """A Sequential around a layer: the same gradients as the layer alone, each within bf16's rounding."""
+    m = _small()
+    x = torch.randn(2, 70, 256, device="cuda").bfloat16()
+    dy = torch.randn_like(x)
+    want = torch.autograd.grad(m(x)[0], list(m.parameters()), dy)
+    calls = []
+    m._modules[name] = torch.nn.Sequential(m._modules[name])
+    m._modules[name].register_forward_hook(lambda *a: calls.append(1))
+    for amp in (False, True):
+        with torch.autocast("cuda", torch.bfloat16, enabled=amp):
+            y = m(x)[0]
+        for a, b in zip(torch.autograd.grad(y, list(m.parameters()), dy), want):
+            assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
+    assert len(calls) == 2

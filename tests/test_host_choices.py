@@ -300,3 +300,16 @@ def test_contiguous_rows_off_the_alignment_are_copied():
     assert kernels.weight_grad_rows(flat[1:129].view(8, 16)).data_ptr() % 16 == 0
     whole = flat[8:136].view(8, 16)
     assert kernels._aligned4(whole, 8) is whole
+
+
+def test_training_branch_asks_replaced_layers_nothing_but_their_call(monkeypatch):
+    # a Sequential around a layer has neither in_features nor a weight
+    from transformer_amd import MLA, ModelArgs, training
+    monkeypatch.setattr(training, "plain_call", lambda *t: True)  # (CPU tensors)
+    for name in ("q_up", "k_up", "v_up"):
+        m = MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=64)).to(torch.bfloat16)
+        d = torch.zeros(1, 4, 128 + 4 * 64 + 128, dtype=torch.bfloat16)
+        assert training.takes_attention(m, d)
+        m._modules[name] = torch.nn.Sequential(m._modules[name])
+        assert not training.takes_attention(m, d)
+        assert not training.takes(m._modules[name], d[..., :128])

@@ -205,13 +205,14 @@ def takes_attention(mla, d: torch.Tensor) -> bool:
     """Whether ``attention`` may run the no-cache branch on the down-projections' bf16 output ``d``: its gradient or a
     weight's is needed, the three layers are plain in bf16 arithmetic, and every part of ``d`` is whole 16-byte runs."""
     mods = [mla._modules[n] for n in ("q_up", "k_up", "v_up")]
+    # (plain layers first: nothing else is known to have a weight)
     if not (torch.is_grad_enabled() and d.dtype == torch.bfloat16 and d.numel() > 0
+            and all(_bf16_arithmetic(m, d) for m in mods)
             and mla.d_latent % 8 == 0 and mods[0].in_features % 8 == 0
             and mla.content_dim in kernels.SUPPORTED_NOPE and mla.v_head_dim in kernels.SUPPORTED_V):
         return False
-    ws = [m._parameters.get("weight") for m in mods]
-    return (all(w is not None for w in ws) and (d.requires_grad or any(w.requires_grad for w in ws))
-            and all(_bf16_arithmetic(m, d) for m in mods) and plain_call(d, *ws))
+    ws = [m.weight for m in mods]
+    return (d.requires_grad or any(w.requires_grad for w in ws)) and plain_call(d, *ws)
 
 
 def attention(mla, d: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
