@@ -209,3 +209,32 @@ def test_replaced_layers_train_through_their_own_call(name):
         for a, b in zip(torch.autograd.grad(y, list(m.parameters()), dy), want):
             assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
     assert len(calls) == 2
+
+
+def test_undefined_gradients_give_zeros():
+    """A consumer whose backward returns None: each operator's and the training branch's gradients are zeros."""
+    import math
+    from transformer_amd import RMSNorm, kernels, training
+
+    class NoGrad(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x + 1
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    r = lambda *s: torch.randn(*s, device="cuda").bfloat16().requires_grad_(True)
+    m, norm = _small(), RMSNorm(256).cuda()
+    x, qk = r(1, 40, 256), r(1, 40, 3, 64)
+    q, k, v = r(1, 40, 2, 64), r(1, 40, 2, 64), r(1, 40, 2, 128)
+    cos, sin = m.rope.cos_cached, m.rope.sin_cached
+    scale = 1 / math.sqrt(128)
+    calls = [(kernels.eager.rope(qk, cos, sin, 0, False), [qk]), (norm(x), [x, norm.weight]),
+             (kernels.eager.prefill_fwd(q, r(1, 40, 2, 64), k, r(1, 40, 2, 64), v, scale, True, 0)[0], [q, k, v]),
+             (kernels.eager.prefill_fwd_rope(q, r(1, 40, 2, 64), k, r(1, 40, 2, 64), v, cos, sin, scale, True, 0, 0,
+                                             True)[0], [q, k, v]),
+             (training.linear(x, m.o_proj.weight), [x, m.o_proj.weight]), (m(x)[0], [x] + list(m.parameters()))]
+    for y, leaves in calls:
+        assert all(g is not None and not g.any() for g in torch.autograd.grad(NoGrad.apply(y).sum(), leaves))

@@ -313,3 +313,45 @@ def test_training_branch_asks_replaced_layers_nothing_but_their_call(monkeypatch
         m._modules[name] = torch.nn.Sequential(m._modules[name])
         assert not training.takes_attention(m, d)
         assert not training.takes(m._modules[name], d[..., :128])
+
+
+@pytest.mark.parametrize("n_outputs", [1, 3])
+def test_undefined_gradients_reach_the_formulas_as_zeros(monkeypatch, n_outputs):
+    # a consumer whose backward returns None leaves the gradient undefined: the registered operators' autograd makes zeros
+    # of it, and so does the autograd.Function in their place (of the first output alone: the others have no gradient)
+    from transformer_amd import kernels
+    seen = []
+
+    def body(x):
+        y = x * 2
+        return y if n_outputs == 1 else (y, x.sum(), x.amax())
+
+    def setup(ctx, inputs, output):
+        if n_outputs > 1:
+            ctx.mark_non_differentiable(*output[1:])
+
+    def backward(ctx, grad, *others):
+        assert not kernels.batched_grad(grad)
+        seen.append((grad.clone(), others))
+        return grad * 2
+
+    monkeypatch.setitem(kernels._BODIES, "probe", body)
+    monkeypatch.setitem(kernels._FORMULAS, "probe", (setup, backward))
+    fn = kernels._function("probe")
+
+    class NoGrad(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x + 1
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    for wrap, want in ((NoGrad.apply, 0.0), (lambda t: t + 1, 1.0)):
+        x = torch.ones(2, 3, requires_grad=True)
+        y = fn.apply(x)
+        wrap(y if n_outputs == 1 else y[0]).sum().backward()
+        grad, others = seen.pop()
+        assert torch.equal(grad, torch.full((2, 3), want)) and all(o is None for o in others)
+        assert torch.equal(x.grad, 2 * grad)

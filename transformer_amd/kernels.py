@@ -1093,11 +1093,19 @@ def _function(name: str):
 
     def setup_context(ctx, inputs, output):
         ctx.set_materialize_grads(False)
+        o = output[0] if isinstance(output, tuple) else output  # the one that has a gradient
+        ctx.output_like = o.shape, o.dtype, o.device
         setup(ctx, inputs, output)
+
+    def run_backward(ctx, grad, *others):
+        if grad is None:  # undefined (a consumer's backward returned None): zeros, as under the operator
+            shape, dtype, device = ctx.output_like
+            grad = torch.zeros(shape, dtype=dtype, device=device)
+        return backward(ctx, grad, *others)
 
     return type("_" + name, (torch.autograd.Function,), {
         "forward": staticmethod(forward), "setup_context": staticmethod(setup_context),
-        "backward": staticmethod(backward)})
+        "backward": staticmethod(run_backward)})
 
 
 def _eager_call(name: str):
