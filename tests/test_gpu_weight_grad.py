@@ -238,3 +238,31 @@ def test_undefined_gradients_give_zeros():
              (training.linear(x, m.o_proj.weight), [x, m.o_proj.weight]), (m(x)[0], [x] + list(m.parameters()))]
     for y, leaves in calls:
         assert all(g is not None and not g.any() for g in torch.autograd.grad(NoGrad.apply(y).sum(), leaves))
+
+
+@pytest.mark.parametrize("tied", [False, True])
+def test_operator_backward_of_the_attention_sees_the_weights_of_the_forward(tied):
+    """fp32 weights under autocast, written between forward and backward: a batch of gradients and create_graph use the
+    forward's values as the plain backward does (the two ways round at other places: as many roundings of 2^-9 as in
+    test_batched_gradients_through_the_training_branch), also where k_up and v_up are one weight."""
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(9)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs(d_model=256, n_heads=2, head_dim=192, d_latent=128, q_lora_rank=128, qk_nope_dim=128,
+                          v_head_dim=128, max_seq_len=128))
+    if tied:
+        m.v_up.weight = m.k_up.weight
+    x = torch.randn(1, 70, 256, device="cuda").requires_grad_(True)
+    dy = torch.randn(1, 70, 256, device="cuda").bfloat16()
+    leaves = [x] + list(m.parameters())
+    with torch.autocast("cuda", torch.bfloat16):
+        y = m(x)[0]
+    want = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.mul_(2)
+    batched = [t[0] for t in torch.autograd.grad(y, leaves, dy[None], is_grads_batched=True, retain_graph=True)]
+    for got in (torch.autograd.grad(y, leaves, dy, retain_graph=True), batched,
+                torch.autograd.grad(y, leaves, dy, create_graph=True)):
+        for a, b in zip(got, want):
+            assert (a.double() - b.double()).norm() <= 6 * 2.0 ** -9 * b.double().norm()

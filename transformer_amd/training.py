@@ -90,6 +90,21 @@ def _by_operators(grad) -> bool:
     return torch.is_grad_enabled() or kernels.batched_grad(grad) or kernels._not_plain((grad,))
 
 
+class _Kept(torch.autograd.Function):
+    """The forward's copy of ``weights`` (their rows below each other, cast), whose gradient goes to the weights: an
+    operator backward sees the values that the forward saw, whatever has been written to the weights since."""
+
+    @staticmethod
+    def forward(ctx, W, *weights):
+        ctx.parts = [(w.size(0), w.dtype) for w in weights]
+        return W.view_as(W)
+
+    @staticmethod
+    def backward(ctx, g):
+        rows = g.split([n for n, _ in ctx.parts])
+        return (None, *(r.to(dt) for r, (_, dt) in zip(rows, ctx.parts)))
+
+
 def on_rows(product, x, W):
     """``product(x, W) [rows, N]`` over x's rows as one matrix.  torch's own product of a batch whose rows are not evenly
     spaced (a slice of longer sequences, a transpose) with a weight that needs no gradient is a batched one over the
@@ -113,7 +128,7 @@ class _Linear(torch.autograd.Function):
         weights = ctx.weights
         dy2, x2 = dy.reshape(-1, dy.size(-1)), x.reshape(-1, x.size(-1))
         if _by_operators(dy):  # torch's operators on the inputs
-            W = torch.cat(weights, 0).to(x.dtype)
+            W = _Kept.apply(W, *weights)
             dx = torch.matmul(dy2, W).view(x.shape)
             dW = torch.matmul(dy2.t(), x2)
             return (dx, None) + tuple(g.to(w.dtype) for g, w in zip(dW.split([w.size(0) for w in weights]), weights))
@@ -159,11 +174,17 @@ class _Attention(torch.autograd.Function):
         H, dn, dv, hr, ql, dl = ctx.layout
         B, T, n = d.shape
         if _by_operators(do):
-            inputs = [t for t, need in zip((d, *ctx.weights), ctx.needs_input_grad) if need]
             with torch.enable_grad():
-                out = _attention_by_operators(d, *ctx.weights, cos, sin, ctx.layout, ctx.scale)
-            got = iter(torch.autograd.grad(out, inputs, do, create_graph=torch.is_grad_enabled()))
-            return tuple(next(got) if need else None for need in ctx.needs_input_grad[:4]) + (None,) * 4
+                Wq, Wkv = _Kept.apply(Wqb, ctx.weights[0]), _Kept.apply(Wkv, *ctx.weights[1:])
+                out = _attention_by_operators(d, Wq, Wkv, cos, sin, ctx.layout, ctx.scale)
+            # (with respect to the copies: k_up and v_up may be one tied weight)
+            got = iter(torch.autograd.grad(out, [t for t in (d, Wq, Wkv) if t.requires_grad], do,
+                                           create_graph=torch.is_grad_enabled()))
+            gd, gq, gkv = (next(got) if t.requires_grad else None for t in (d, Wq, Wkv))
+            gk, gv = gkv.split([H * dn, H * dv]) if gkv is not None else (None, None)
+            grads = [g.to(w.dtype) if need else None
+                     for g, w, need in zip((gq, gk, gv), ctx.weights, ctx.needs_input_grad[1:4])]
+            return (gd, *grads) + (None,) * 4
         d2 = d.reshape(B * T, n)
         dd = torch.empty(B * T, n, dtype=d.dtype, device=d.device)
         dqk = dd[:, ql:n - dl].view(B, T, H + hr, 64)
@@ -189,13 +210,14 @@ def _kv_views(kv, B, T, H, dn, dv):
     return kv[:, :H * dn].view(B, T, H, dn), kv[:, H * dn:].view(B, T, H, dv)
 
 
-def _attention_by_operators(d, Wq, Wk, Wv, cos, sin, layout, scale):
+def _attention_by_operators(d, Wq, Wkv, cos, sin, layout, scale):
     H, dn, dv, hr, ql, dl = layout
     B, T, n = d.shape
     q_low, qk, kv = d.split([ql, (H + hr) * 64, dl], -1)
     lin = torch.nn.functional.linear
     qk = qk.view(B, T, H + hr, 64)
-    q, k, v = (lin(t, w.to(d.dtype)).view(B, T, H, -1) for t, w in ((q_low, Wq), (kv, Wk), (kv, Wv)))
+    Wk, Wv = Wkv.split([H * dn, H * dv])
+    q, k, v = (lin(t, w).view(B, T, H, -1) for t, w in ((q_low, Wq), (kv, Wk), (kv, Wv)))
     k_rope = kernels.eager.rope(qk[:, :, H:], cos, sin, 0, False)
     o, _, _ = kernels.eager.prefill_fwd_rope(q, qk[:, :, :H], k, k_rope, v, cos, sin, scale, True, 0, 0, True)
     return o.reshape(B, T, H * v.size(-1))
