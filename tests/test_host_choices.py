@@ -355,3 +355,24 @@ def test_undefined_gradients_reach_the_formulas_as_zeros(monkeypatch, n_outputs)
         grad, others = seen.pop()
         assert torch.equal(grad, torch.full((2, 3), want)) and all(o is None for o in others)
         assert torch.equal(x.grad, 2 * grad)
+
+
+def test_autocast_does_not_cast_float64_inputs(monkeypatch):
+    # torch's layers refuse a float64 (or integer) input beside autocast's bf16 weight, and the training branch leaves it to them
+    from transformer_amd import MLA, ModelArgs, training
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *a: True)  # (no GPU: torch turns autocast off)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda *a: torch.bfloat16)
+    monkeypatch.setattr(training, "plain_call", lambda *t: True)
+    taken = []
+    monkeypatch.setattr(training, "linear", lambda x, *ws, **k: taken.append(x.dtype))
+    m = MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=64))
+    for dt in (torch.bfloat16, torch.float32, torch.float64, torch.int32):
+        x = torch.zeros(2, 3, 256, dtype=dt)
+        ok = dt in (torch.bfloat16, torch.float32)
+        assert training.takes(m.o_proj, x) == ok
+        if ok:
+            m._down_all(x)
+        else:
+            with pytest.raises(RuntimeError):
+                m._down_all(x)
+    assert taken == [torch.bfloat16] * 2

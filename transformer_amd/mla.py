@@ -339,7 +339,8 @@ class MLA(nn.Module):
             # 214 against 243 us at the benchmark down-projections), whose products are single ones
             dt = torch.get_autocast_dtype("cuda") if amp else \
                 torch.promote_types(torch.promote_types(ws[0].dtype, ws[1].dtype), ws[2].dtype)
-            if (split or (dt == torch.bfloat16 and (amp or x.dtype == dt))) and training.plain_call(x, *ws):
+            if (split or (dt == torch.bfloat16 and (x.dtype in training._AUTOCAST_INPUTS if amp else x.dtype == dt))) \
+                    and training.plain_call(x, *ws):
                 return training.linear(x.to(dt), *ws, product=_down_product)
             return torch.nn.functional.linear(x, torch.cat(ws, 0))
         dt = torch.get_autocast_dtype("cuda") if amp else ws[0].dtype

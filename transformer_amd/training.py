@@ -44,12 +44,16 @@ def takes(m: nn.Module, x: torch.Tensor) -> bool:
             and plain_call(x, w))
 
 
+_AUTOCAST_INPUTS = (torch.bfloat16, torch.float16, torch.float32)  # what autocast casts (float64 it leaves)
+
+
 def _bf16_arithmetic(m: nn.Module, x: torch.Tensor) -> bool:
     if not plain_linear(m):
         return False
     w = m._parameters["weight"]
     if torch.is_autocast_enabled("cuda"):
-        return torch.get_autocast_dtype("cuda") == torch.bfloat16 and w.dtype in (torch.bfloat16, torch.float32)
+        return torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.dtype in _AUTOCAST_INPUTS \
+            and w.dtype in (torch.bfloat16, torch.float32)
     return w.dtype == torch.bfloat16 and x.dtype == w.dtype
 
 
