@@ -116,3 +116,33 @@ def test_few_row_calls_run_hooked_projections(B, T, L, dims):
         want = m(x, cache, True)[0]
         hook.remove()
     assert len(seen) == 2 and torch.equal(y, want)
+
+
+@pytest.mark.parametrize("weights", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [9, 75])
+def test_chunk_sees_updates_past_the_version_counter(T, weights):
+    """p.data writes do not count in p._version.  A chunk over per-head K and V reads q_up, k_up, v_up and o_proj
+    themselves: doubling v_up so doubles the attention's output, exactly, and the layer's with it."""
+    from contextlib import nullcontext
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(10)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs())  # bf16 RoPE tables
+        m = m.to(weights) if weights == torch.bfloat16 else m
+        x = torch.randn(2, T, m.d_model).to(weights)
+        cache = {"latent": torch.randn(2, 40, m.d_latent).bfloat16(),
+                 "k_rope": torch.randn(2, m.n_k_rope_heads, 40, 64).bfloat16(), "seq_len": 40}
+    amp = nullcontext() if weights == torch.bfloat16 else torch.autocast("cuda", torch.bfloat16, cache_enabled=False)
+    with torch.no_grad(), amp:
+        y = m(x, dict(cache), True)[0]
+        for name in ("v_up", "o_proj"):
+            m._modules[name].weight.data.mul_(2)
+            y2 = m(x, dict(cache), True)[0]
+            assert torch.equal(y2, 2 * y), name
+            y = y2
+        for name in ("q_up", "k_up"):  # other scores
+            m._modules[name].weight.data.mul_(2)
+            y2 = m(x, dict(cache), True)[0]
+            assert not torch.equal(y2, y), name
+            y = y2
+    assert "kv_up" not in m.__dict__.get("_derived", {})

@@ -174,7 +174,8 @@ def test_expanded_gradients_and_overlapping_inputs(B, weights):
     from transformer_amd import MLA, ModelArgs
     torch.manual_seed(8)
     with torch.device("cuda"):
-        m = MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=128)).to(weights)
+        m = MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=128))  # bf16 RoPE tables
+    m = m.to(weights) if weights == torch.bfloat16 else m
     base = torch.randn(256 * 80, device="cuda").bfloat16()
     col = torch.randn(256, device="cuda").bfloat16()
     inputs = [base.as_strided((B, 37, 256), (128, 256, 1)), base.as_strided((B, 37, 256), (8, 128, 1)),

@@ -192,7 +192,7 @@ class MLA(nn.Module):
         """A derived weight (``make()``, cast to ``dtype``) kept while the parameters it reads
         are unchanged (same storage and version counter); autograd off only."""
         params = [self.q_down.weight, self.qk_rope.weight, self.kv_down.weight] if name == "down" else \
-            [self.k_up.weight, self.v_up.weight] if name == "kv_up" else [getattr(self, name.split(":")[0]).weight]
+            [getattr(self, name.split(":")[0]).weight]
         key = tuple((w.data_ptr(), w._version) for w in params) + (dtype,)
         cache = self.__dict__.setdefault("_derived", {})
         hit = cache.get(name)
@@ -357,10 +357,8 @@ class MLA(nn.Module):
 
     def _kv_up_as_one(self, kv_latent):
         """Whether ``k_up`` and ``v_up`` over a cache may be one bf16 product: autograd off, both plain layers in bf16
-        arithmetic, eager.  Not in a capture: a recorded call reads the weights themselves, so a replay sees them as
-        they then are."""
+        arithmetic, eager."""
         return (not torch.is_grad_enabled() and kv_latent.dtype == torch.bfloat16
-                and not torch.cuda.is_current_stream_capturing()
                 and all(training._bf16_arithmetic(self._modules[n], kv_latent) for n in ("k_up", "v_up"))
                 and training.plain_call(kv_latent))
 
@@ -525,10 +523,9 @@ class MLA(nn.Module):
         else:
             # T > 1 with the bottom-right causal mask of :273-281 (q_offset = pos_offset)
             if self._kv_up_as_one(kv_latent):
-                # K and V as the column views of one product over weights kept in bf16: the latent rows are read once, and
-                # the launches bound a chunk (B = 4, T = 75 over 2500, default dims, fp32 weights: 278 -> 257 us)
-                W = self._cached_weight("kv_up", lambda: torch.cat([self.k_up.weight, self.v_up.weight], 0),
-                                        torch.bfloat16)
+                # K and V as the column views of one product: the latent rows are read once.  The weights are joined on
+                # every call: kept copies would miss an update through p.data, and a recorded call any update
+                W = torch.cat([self.k_up.weight, self.v_up.weight], 0).to(torch.bfloat16)
                 kv = torch.mm(kv_latent.reshape(B * kv_len, self.d_latent), W.t())
                 k_nope, v = training._kv_views(kv, B, kv_len, H, dn, dv)
             else:
