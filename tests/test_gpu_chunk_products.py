@@ -146,3 +146,44 @@ def test_chunk_sees_updates_past_the_version_counter(T, weights):
             assert not torch.equal(y2, y), name
             y = y2
     assert "kv_up" not in m.__dict__.get("_derived", {})
+
+
+@pytest.mark.parametrize("weights", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,L", [(2, 20, None), (2, 100, 0), (2, 10, 40), (2, 70, 40), (2, 1, 40)])
+def test_compiled_calls_are_one_graph_at_the_default_dims(B, T, L, weights):
+    """No-cache, prompt, chunks on either side of 64 rows, one token; fullgraph raises at a graph break.  Compiled calls take
+    the layers where eager ones may take the few-row kernels: a few roundings of 2^-9."""
+    from contextlib import nullcontext
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(11)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs())  # bf16 RoPE tables
+        m = m.to(weights) if weights == torch.bfloat16 else m
+        x = torch.randn(B, T, m.d_model).to(weights)
+        cache = None
+        if L:
+            cache = {"latent": torch.randn(B, L, m.d_latent).bfloat16(),
+                     "k_rope": torch.randn(B, m.n_k_rope_heads, L, 64).bfloat16(), "seq_len": L}
+    amp = nullcontext() if weights == torch.bfloat16 else torch.autocast("cuda", torch.bfloat16)
+    torch._dynamo.reset()
+    with torch.no_grad(), amp:
+        got = torch.compile(lambda t: m(t, cache, L is not None)[0], backend="eager", fullgraph=True)(x)
+        want = m(x, cache, L is not None)[0]
+    assert (got.double() - want.double()).norm() <= 8 * 2.0 ** -9 * want.double().norm()
+
+
+def test_absorbed_chunk_compiles_as_it_runs():
+    """The absorbed form's last product writes a view in eager mode and is a plain product under torch.compile: bit for bit."""
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(12)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs.mla_baseline()).to(torch.bfloat16)
+        x = torch.randn(2, 70, m.d_model).bfloat16()
+        cache = {"latent": torch.randn(2, 40, m.d_latent).bfloat16(), "k_rope": torch.randn(2, 1, 40, 64).bfloat16(),
+                 "seq_len": 40}
+    torch._dynamo.reset()
+    with torch.no_grad():
+        reasons = [str(r.reason) for r in torch._dynamo.explain(lambda t: m(t, cache, True)[0])(x).break_reasons]
+        assert not any("out=" in r for r in reasons), reasons
+        got = torch.compile(lambda t: m(t, cache, True)[0], backend="eager")(x)
+        assert torch.equal(got, m(x, cache, True)[0])

@@ -301,7 +301,8 @@ class MLA(nn.Module):
         """Few-row bf16 products (the decode step): autograd off, at most ROWS_FAST_M rows, bf16 arithmetic (bf16
         weights, or bf16 autocast), and ``q_up`` and ``o_proj`` plain layers: a hooked, wrapped or parametrized one is
         called.  fp32 weights would be read from kept bf16 copies: not in a capture, whose replays would no longer
-        follow the weights, and only where the whole step fits linear_rows."""
+        follow the weights, and only where the whole step fits linear_rows.  Where it does not, torch.compile keeps the
+        layers too: they trace as one graph, the lookup of a kept weight does not."""
         if torch.is_grad_enabled() or x.size(0) * x.size(1) > kernels.ROWS_FAST_M or not self._plain_projections() \
                 or not self._rows_proj_ok():
             return False
@@ -311,7 +312,7 @@ class MLA(nn.Module):
             return False
         whole = kernels.rows_fit(self.content_dim, self.d_latent)
         if wq == torch.bfloat16 and wo == torch.bfloat16:
-            return whole or amp or x.dtype == torch.bfloat16
+            return whole or ((amp or x.dtype == torch.bfloat16) and not torch.compiler.is_compiling())
         return whole and not torch.cuda.is_current_stream_capturing()
 
     def _plain_projections(self):
@@ -517,9 +518,13 @@ class MLA(nn.Module):
             ctx, _ = ops.prefill_cached(q_lat, b(q_rope), b(kv_latent), b(k_pos), pos_offset, self.scale, True)
             Wvt = self._cached_weight("v_up:t", lambda: self.v_up.weight.view(H, dv, DL).transpose(1, 2),
                                       torch.bfloat16)  # [H, DL, dv]
-            out = torch.empty(B * T, H, dv, dtype=torch.bfloat16, device=x.device)
-            torch.bmm(ctx.permute(2, 0, 1, 3).reshape(H, B * T, DL), Wvt, out=out.transpose(0, 1))
-            out = out.view(B, T, H * dv).to(cdt)
+            ctx = ctx.permute(2, 0, 1, 3).reshape(H, B * T, DL)
+            if torch.compiler.is_compiling():  # (dynamo breaks its graph at out= of a view)
+                out = torch.bmm(ctx, Wvt).transpose(0, 1).reshape(B, T, H * dv).to(cdt)
+            else:
+                out = torch.empty(B * T, H, dv, dtype=torch.bfloat16, device=x.device)
+                torch.bmm(ctx, Wvt, out=out.transpose(0, 1))
+                out = out.view(B, T, H * dv).to(cdt)
         else:
             # T > 1 with the bottom-right causal mask of :273-281 (q_offset = pos_offset)
             if self._kv_up_as_one(kv_latent):
