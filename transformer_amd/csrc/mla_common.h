@@ -20,6 +20,7 @@
 #include <stdint.h>
 
 #include "../../include/mla_mi355x.h"
+#include "plans.h"
 
 namespace mla {
 
@@ -226,37 +227,6 @@ int check_operand(const char* op, const char* name, const void* ptr, const mla_s
 // before scaling (a positive factor commutes with max), and 2^(s * scale * log2 e) must
 // stay finite for finite scores
 int check_scale(const char* op, float scale);
-
-// Whether a causal attention kernel's grid runs one tile of 128 rows per workgroup, longest first, instead of mirrored
-// pairs (tiles r and n - 1 - r of one (b, h), always the same work together).  Pairs start a new round of workgroups for
-// any remainder; single tiles fill the chip to the end but start twice as often, without the next tile's prefetch, and
-// share less of a (b, h) in L2.  Results are the same bit for bit.  Times in units of a pair's, n_bh (b, h) of n tiles:
-//   single tiles: the work over the workgroups that run at once, plus what the starts cost, at least the longest tile;
-//   pairs: whole rounds; where two workgroups share a CU, a last round of one per CU takes a fraction of that.
-// Measured, pairs -> single (us; 14 heads of 64 + 64 or 16 of 128 + 64, B x T), forward / whole backward:
-//   3 x 3000 180 -> 144 / 530 -> 468;  2 x 2600 76 -> 63 / 263 -> 191;  4 x 2900 148 -> 130 / 450 -> 418;  3 x 1900 60 ->
-//   52 / 206 -> 169;  but whole rounds: 12 x 2048 265 -> 279 / 911 -> 990;  4 x 4096 319 -> 320 / 1060 -> 1076.
-struct TileGrid {
-  int64_t n_bh, n;
-  bool square;  // causal from the first key: tile sizes 1 .. n, else alike
-  double longest() const { return square ? (double)n / (double)(n + 1) : 0.5; }
-  double work() const { return (double)n_bh * (double)n / 2; }
-  int64_t pairs() const { return n_bh * ((n + 1) / 2); }
-};
-inline bool single_tiles_one_per_cu(const TileGrid& g) {  // 256 workgroups at once
-  if (g.n < 2) return false;
-  const double pair = (double)((g.pairs() + 255) / 256);
-  const double most = g.work() / 256 * (1.0 + 1.0 / (double)g.n), single = most > g.longest() ? most : g.longest();
-  return single < 0.97 * pair;
-}
-inline bool single_tiles_two_per_cu(const TileGrid& g) {  // 512, two on a CU
-  if (g.n < 2) return false;
-  const int64_t rest = g.pairs() % 512;
-  const double last = rest == 0 ? 0.0 : rest > 256 ? 1.0 : 0.42 + (rest > 160 ? 0.25 * (double)(rest - 160) / 96 : 0.0);
-  const double pair = (double)(g.pairs() / 512) + last;
-  const double most = g.work() / 512 * (1.0 + 0.6 / (double)g.n), low = 0.8 * g.longest();
-  return (most > low ? most : low) < 0.95 * pair;
-}
 }  // namespace mla
 
 #define MLA_TRY(expr)              \

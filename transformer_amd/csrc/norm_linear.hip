@@ -23,7 +23,7 @@
 //   * the one barrier of a stage lies between its two 16-wide halves: the first half's products run under the second
 //     half's reads and the normalisation, the next stage's first reads under the second half's products, and the steady
 //     loop has no branch.  With one barrier at the end of a stage every read waited behind it;
-//   * the tile is chosen for the rounds of 256 workgroups (nl_plan below): M = 24576, N = 2624 made 1056 tiles of
+//   * the tile is chosen for the rounds of 256 workgroups (nl_plan in plans.h): M = 24576, N = 2624 made 1056 tiles of
 //     256 x 256, a fifth round of 32 workgroups, where the last 64 columns are now tiles of their own, a quarter as long.
 // Measured calls (the row pass included), before -> now: 24576 x 2624 x 2048 388 -> 337 us, 12288 x 2560 x 1792 137 -> 129,
 // 6555 x 2496 x 1440 109 -> 89, 2735 x 2000 x 1632 63 -> 38, 1000 x 2624 x 2048 68 -> 39, 700 x 512 x 1056 36 -> 19.
@@ -43,7 +43,6 @@ struct NlParams {
   float inv_k, eps;
 };
 
-constexpr int kNlBK = 32;      // k per stage
 constexpr int kNlStages = 4;   // LDS ring depth
 constexpr int kNlWaves = 8;
 constexpr int kNlMaxK = 4096;
@@ -291,42 +290,6 @@ typedef NlCfg<256, 256, 2> NlWide;   // wave 128 n x 64 m
 typedef NlCfg<128, 256, 2> NlRest;   // wave 64 x 64: an n remainder of up to 128 beside NlWide tiles
 typedef NlCfg<256, 128, 4> NlHalf;   // wave 64 x 64
 typedef NlCfg<128, 128, 4> NlSmall;  // wave 32 n x 64 m
-
-struct NlPlan {
-  int kind;  // 0 NlWide (+ NlRest), 1 NlHalf, 2 NlSmall
-  int64_t n_nt, n_wide, n_rest;
-};
-
-// The least of: rounds of 256 workgroups (one per CU) x (the tile's time per stage x stages + what a workgroup takes
-// beside them), both fitted to the measured calls (us at M x N x K, wide / half / small tiles): 12288 x 2560 x 1792 129.0 /
-// 146.0 / 168.8 (two full rounds of wide tiles), 8192 x 2624 x 2048 132.8 / 127.7 / 140.7, 2735 x 2000 x 1632 57.1 / 36.6 /
-// 40.2, 1000 x 2624 x 2048 61.7 / 42.6 / 39.3 (wide tiles leave most of the chip idle).  Small tiles share a CU.
-static NlPlan nl_plan(int64_t M, int64_t N, int64_t K) {
-  NlPlan best{};
-  double best_t = 1e300;
-  const double stages = (double)(K / kNlBK);
-  static const int bn[3] = {256, 256, 128}, bm[3] = {256, 128, 128};
-  static const double ts[3] = {1.0, 0.6, 0.39}, fixed[3] = {6.0, 4.0, 1.5};
-  for (int kind = 0; kind < 3; ++kind) {
-    const int64_t mt = (M + bm[kind] - 1) / bm[kind];
-    int64_t nt = (N + bn[kind] - 1) / bn[kind], rest = 0;
-    if (kind == 0 && nt > 1 && N % 256 != 0 && N % 256 <= 128) {
-      --nt;
-      rest = mt;
-    }
-    const int64_t wide = mt * nt;
-    // the remainder's tiles fill the last round's free CUs first
-    double rounds = (double)((wide + 255) / 256);
-    const int64_t over = rest - (int64_t)(rounds * 256 - wide);
-    if (over > 0) rounds += 0.6 * (double)((over + 255) / 256);
-    const double t = rounds * (stages * ts[kind] + fixed[kind]);
-    if (t < best_t) {
-      best_t = t;
-      best = NlPlan{kind, nt, wide, rest};
-    }
-  }
-  return best;
-}
 
 }  // namespace mla
 

@@ -28,7 +28,7 @@
 //     S^T (32k x 32q) = K . Q^T,  dP^T = V . dO^T   (lanes own a query)
 //     dQ^T (DQK x 32q) += K^T . dS^T                (K^T by transpose read)
 // Workgroups take mirrored pairs of tiles of one (b, h) so causal work is balanced, or single tiles, longest first, where
-// pairs would leave much of a last round empty (TileGrid in mla_common.h).
+// pairs would leave much of a last round empty (TileGrid in plans.h).
 #include <type_traits>
 
 #include "mla_common.h"

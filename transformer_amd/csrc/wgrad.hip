@@ -15,7 +15,7 @@
 //
 // Few weights have as many 256 x 256 tiles as the chip has CUs, so the tokens are cut into S segments and a second
 // kernel adds the segments' fp32 partials in order (no atomics: the result is bitwise reproducible).  S and the tile
-// come from a cost model (wg_plan below).
+// come from a cost model (wg_plan in plans.h).
 //
 // Measured (kernel trace, main + segment sum, against the library's product over the same operands):
 //   M = 12288, N x K = 2560 x 1792: 106.5 + 11.8 us (main 1059 TFLOP/s) against 219.6
@@ -44,7 +44,6 @@ struct WgParams {
   int out_f32;
 };
 
-constexpr int kWgSt = 32;     // tokens per stage
 constexpr int kWgRing = 4;    // stages
 constexpr int kWgWaves = 8;
 
@@ -274,40 +273,6 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(WgParams p) {
 
 typedef WgCfg<256, 256, 2> WgWide;    // wave 128 x 64
 typedef WgCfg<256, 128, 4> WgNarrow;  // wave 64 x 64
-
-struct WgPlan {
-  int narrow, S, seg, nt, kt;
-  int64_t part_bytes;
-};
-
-// The plan of least estimated time: rounds of 256 workgroups (one per CU), each its stages at the measured 1.05 us (wide
-// tile: 128 stages of 4096 x 2048 took 124-134 us) or 0.62 us (narrow) plus 4 us of start and stores, and where the
-// tokens are cut the second kernel with its partials at 4 TB/s.  Wide tiles stage fewer bytes per product, so they win
-// where the weight has enough of them; narrow ones (and more segments) where it has few: 896 x 384 makes 12.
-static WgPlan wg_plan(int64_t M, int64_t N, int64_t K) {
-  WgPlan best{};
-  double best_t = 1e300;
-  const int64_t st = (M + kWgSt - 1) / kWgSt;
-  for (int narrow = 0; narrow < 2; ++narrow) {
-    const int64_t TN = 256, TK = narrow ? 128 : 256;
-    const int64_t nt = (N + TN - 1) / TN, kt = (K + TK - 1) / TK, tiles = nt * kt;
-    const double ts = narrow ? 0.62 : 1.05;  // us per stage of a workgroup
-    for (int64_t S = 1; S <= 32 && S <= st; ++S) {
-      const int64_t per = (st + S - 1) / S;
-      if ((st + per - 1) / per != S) continue;  // fewer segments hold the same stages
-      const double rounds = (double)((tiles * S + 255) / 256);
-      double t = rounds * ((double)per * ts + 4.0);
-      const int64_t pb = S > 1 ? tiles * S * TN * TK * 4 : 0;
-      if (S > 1) t += 4.0 + (double)pb / 4.0e6;
-      if (pb > (256ll << 20)) continue;
-      if (t < best_t) {
-        best_t = t;
-        best = WgPlan{narrow, (int)S, (int)(per * kWgSt), (int)nt, (int)kt, pb};
-      }
-    }
-  }
-  return best;
-}
 
 static int wg_check(const mla_weight_grad_args* a) {
   const char* op = "mla_weight_grad";
