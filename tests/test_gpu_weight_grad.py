@@ -2,22 +2,31 @@
 import pytest
 import torch
 
+from tests import plans
+
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("out_fp32", [True, False])
-@pytest.mark.parametrize("M,N,K,pad", [
-    (1, 8, 8, 0),            # one token, one 16-byte chunk
-    (31, 264, 136, 0),       # a ragged only stage, past one tile both ways
-    (32, 256, 128, 8),       # one full stage, strided rows
-    (33, 256, 256, 0),       # a one-token tail
-    (97, 1000, 392, 24),     # four stages (the ring's depth) with a tail
-    (160, 256, 256, 0),      # five stages: one through the steady loop
-    (1000, 2624, 2048, 0),   # one segment of wide or narrow tiles
-    (4100, 384, 1792, 16),   # many segments, the last one ragged
-    (12288, 896, 384, 0),    # the segments' partials read eight at a time, and a remainder
+@pytest.mark.parametrize("M,N,K,pad,narrow,S", [  # narrow, S: the tile and the token segments that the sizes take
+    (1, 8, 8, 0, 1, 1),             # one token, one 16-byte chunk
+    (31, 264, 136, 0, 1, 1),        # a ragged only stage, past one tile both ways
+    (32, 256, 128, 8, 1, 1),        # one full stage, strided rows
+    (33, 256, 256, 0, 1, 1),        # a one-token tail
+    (97, 1000, 392, 24, 1, 1),      # four stages (the ring's depth) with a tail
+    (160, 256, 256, 0, 1, 1),       # five stages: one through the steady loop
+    (1000, 2624, 2048, 0, 1, 1),    # one segment, 176 narrow tiles
+    (4100, 384, 1792, 16, 1, 9),    # many segments, the last one ragged
+    (12288, 896, 384, 0, 1, 21),    # the segments' partials read eight at a time, and a remainder
+    (33, 1800, 4104, 0, 0, 1),      # wide tiles, ragged both ways, a one-token tail
+    (97, 1800, 4104, 16, 0, 1),     # wide tiles, four stages with a tail
+    (129, 1800, 4104, 0, 0, 1),     # wide tiles, five stages
+    (3001, 2056, 1800, 8, 0, 3),    # wide tiles in segments, ragged both ways, the last one shorter with a tail
+    (6150, 2600, 2056, 0, 0, 2),    # the same, six tokens in the last stage
 ])
-def test_weight_grad_matches_fp64(M, N, K, pad, out_fp32):
+def test_weight_grad_matches_fp64(M, N, K, pad, narrow, S, out_fp32):
+    plan = plans.weight_grad(M, N, K)
+    assert (plan.narrow, plan.S) == (narrow, S), plan
     from transformer_amd import kernels
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     by = torch.randn(M, N + 2 * pad, generator=g, device="cuda").bfloat16()
@@ -62,8 +71,8 @@ def test_weight_grad_rejects_what_it_does_not_take():
 @pytest.mark.parametrize("frozen", [(), ("q_up", "kv_down"), ("q_down", "qk_rope", "kv_down"), ("k_up",)])
 @pytest.mark.parametrize("shared", [False, True])
 def test_module_gradients_equal_torch_layers(monkeypatch, amp, frozen, shared):
-    """The training branch's linear layers against the same module on torch's own (what a hook on each makes it take),
-    for fp32 weights under autocast and bf16 weights, with frozen weights: each gradient within bf16's rounding."""
+    """The training branch's linear layers against the same module on torch's own (plain_call false: what tracing, a mode
+    or a transform makes it take), for fp32 weights under autocast and bf16 weights, with frozen weights: each gradient within bf16's rounding."""
     from transformer_amd import MLA, ModelArgs, training
     g = torch.Generator(device="cuda").manual_seed(3)
     with torch.device("cuda"):
