@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from oracle import mla_oracle as O
+from tests import plans
 from tests.gpu_util import randn_bf16
 
 pytestmark = pytest.mark.gpu
@@ -122,15 +123,22 @@ def test_norm_linear_rejects_bad_shapes(ops):
                         1e-6)
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (6391, 2600, 32),   # 256 x 256 tiles beside a 40-column remainder's tiles; one stage
-    (6391, 2600, 128),  # the ring's four stages
-    (6391, 2600, 160),  # five: one through the steady loop
-    (6391, 2500, 96),   # 256 x 256 tiles, the last column of them ragged
-    (2735, 2000, 512),  # 256 x 128 tiles, ragged both ways
-    (1100, 1304, 544),  # 128 x 128 tiles, ragged both ways
+@pytest.mark.parametrize("M,N,K,kind,rest", [  # the tile that the sizes take, and whether the n remainder has tiles of its own
+    (6391, 2600, 32, plans.NL_SMALL, False),    # 128 x 128 tiles, ragged both ways; one stage
+    (6391, 2600, 128, plans.NL_SMALL, False),   # the ring's four stages
+    (6391, 2600, 160, plans.NL_SMALL, False),   # five: one through the steady loop
+    (6391, 2500, 96, plans.NL_WIDE, False),     # 256 x 256 tiles, the last column of them ragged
+    (2735, 2000, 512, plans.NL_HALF, False),    # 256 x 128 tiles, ragged both ways
+    (1100, 1304, 544, plans.NL_SMALL, False),   # 128 x 128 tiles, 17 stages
+    (14308, 808, 32, plans.NL_WIDE, True),      # 256 x 256 tiles beside a 40-column remainder's, ragged rows; one stage
+    (14308, 868, 128, plans.NL_WIDE, True),     # beside a 100-column remainder's; the ring's four stages
+    (14308, 808, 160, plans.NL_WIDE, True),     # five: one through the steady loop
+    (14308, 896, 192, plans.NL_WIDE, True),     # a remainder of a whole 128 columns; six
+    (14308, 868, 544, plans.NL_WIDE, True),     # 17
 ])
-def test_norm_linear_tile_shapes(ops, M, N, K):
+def test_norm_linear_tile_shapes(ops, M, N, K, kind, rest):
+    plan = plans.norm_linear(M, N, K)
+    assert (plan.kind, plan.n_rest > 0) == (kind, rest), plan
     print(f"case M={M} N={N} K={K}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
