@@ -32,7 +32,7 @@ inline bool single_tiles_one_per_cu(const TileGrid& g) {  // 256 workgroups at o
   const double pair = (double)((g.pairs() + 255) / 256);
   // a start (nothing prefetched) costs a pair's tiles 1 / n of their time; never less than the longest tile
   const double most = g.work() / 256 * (1.0 + 1.0 / (double)g.n), single = most > g.longest() ? most : g.longest();
-  return single < 0.97 * pair;  // (3 %: what runs of one side differ)
+  return single < 0.97 * pair;  // (what is this close stays in pairs)
 }
 inline bool single_tiles_two_per_cu(const TileGrid& g) {  // 512, two on a CU
   if (g.n < 2) return false;

@@ -947,9 +947,18 @@ def weight_grad_fits(M: int, N: int, K: int, dy_stride: int, x_stride: int) -> b
 
 
 def weight_grad(dy: Tensor, x: Tensor, out_fp32: bool = False) -> Tensor:
-    """``dy^T x`` for bf16 ``dy [M, N]`` and ``x [M, K]`` (unit inner stride): the gradient ``[N, K]`` of a linear
+    """``dy^T x`` for bf16 ``dy [M, N]`` and ``x [M, K]``: the gradient ``[N, K]`` of a linear
     layer's weight (the autograd of transformer.py:208-213, :263, :300), fp32 sums, rounded once to bf16 or, with
     ``out_fp32``, not at all.  Not a registered operator: it is called inside backward passes only."""
+    dw = weight_grad_or_none(dy, x, out_fp32)
+    if dw is None:
+        raise ValueError(f"mla_mi355x::weight_grad: dy {tuple(dy.shape)} and x {tuple(x.shape)} with strides "
+                         f"{dy.stride()}, {x.stride()} are outside the kernel's limits")
+    return dw
+
+
+def weight_grad_or_none(dy: Tensor, x: Tensor, out_fp32: bool) -> Optional[Tensor]:
+    """:func:`weight_grad`, or None where the sizes are outside the kernel's limits."""
     op = "mla_mi355x::weight_grad"
     _require_gpu(op, dy, x)
     _bf16(op, dy=dy, x=x)
@@ -959,7 +968,7 @@ def weight_grad(dy: Tensor, x: Tensor, out_fp32: bool = False) -> Tensor:
     (M, N), K = dy.shape, x.size(1)
     sy, sx = (dy.stride(0), x.stride(0)) if M > 1 else (N, K)
     if not weight_grad_fits(M, N, K, sy, sx):
-        raise ValueError(f"{op}: M = {M}, N = {N}, K = {K} with row strides {sy}, {sx} is outside the kernel's limits")
+        return None
     dw = torch.empty(N, K, dtype=torch.float32 if out_fp32 else torch.bfloat16, device=dy.device)
     args = _lib.WeightGradArgs(dy=dy.data_ptr(), x=x.data_ptr(), dw=dw.data_ptr(), workspace=None, workspace_bytes=0,
                                M=M, N=N, K=K, dy_stride=sy, x_stride=sx, dw_stride=K, dw_dtype=_dt_code(dw))

@@ -74,11 +74,7 @@ def weight_grads(dy, x, weights, needed):
     if not any(needed):
         return [None] * len(weights)
     f32 = all(w.dtype == torch.float32 for w in weights)
-    dW = None
-    if dy.dtype == torch.bfloat16:
-        dyr, xr = kernels.weight_grad_rows(dy), kernels.weight_grad_rows(x)
-        if kernels.weight_grad_fits(*dy.shape, x.size(1), dyr.stride(0), xr.stride(0)):
-            dW = kernels.weight_grad(dyr, xr, f32)
+    dW = kernels.weight_grad_or_none(dy, x, f32) if dy.dtype == torch.bfloat16 else None
     if dW is None:
         dW = torch.matmul(dy.t(), x)
     out, r = [], 0
