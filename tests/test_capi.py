@@ -305,3 +305,22 @@ def test_workspace_queries_on_random_sizes(lib):
             a = args[0]._type_()
             fill(a)
             assert f(ctypes.byref(a)) < (1 << 56), name
+
+
+def test_weight_grad_rejects_bad_arguments_without_a_gpu(lib):
+    # each change of a call that is valid (its pointers are never followed: every check precedes the launch)
+    from transformer_amd import _lib
+
+    def args(**change):
+        a = _lib.WeightGradArgs(dy=4096, x=8192, dw=12288, workspace=None, workspace_bytes=0, M=64, N=16, K=24, dy_stride=16,
+                                x_stride=24, dw_stride=24, dw_dtype=_lib.MLA_DTYPE_F32)
+        for k, v in change.items():
+            setattr(a, k, v)
+        return a
+
+    for change in (dict(M=0), dict(M=1 << 24), dict(N=0), dict(N=1 << 20), dict(K=12), dict(N=20), dict(dy=None),
+                   dict(x=8200), dict(dw=12290), dict(dy_stride=8), dict(x_stride=20), dict(dw_stride=16), dict(dw_dtype=7),
+                   dict(dy_stride=1 << 22), dict(x_stride=1 << 25), dict(dy_stride=1 << 61), dict(x_stride=1 << 62),
+                   dict(dy_stride=(1 << 63) - 8), dict(dw_stride=1 << 60), dict(M=100000, workspace=None)):
+        rc = lib.mla_weight_grad(ctypes.byref(args(**change)), None)
+        assert rc in (-1, -2, -3), (change, rc, lib.mla_last_error())

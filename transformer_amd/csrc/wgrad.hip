@@ -288,6 +288,9 @@ static int wg_check(const mla_weight_grad_args* a) {
                 a->x_stride % 8 == 0,
             MLA_ERR_INVALID_ARG, "%s: row strides must cover a row and be multiples of 8 (dy, x)", op);
   MLA_CHECK(a->dw_dtype == MLA_DTYPE_F32 || a->dw_dtype == MLA_DTYPE_BF16, MLA_ERR_UNSUPPORTED, "%s: dw dtype", op);
+  // (before the product below, which a stride near 2^63 would wrap; element offsets of dw stay far below it too)
+  MLA_CHECK(a->dy_stride < (1 << 30) && a->x_stride < (1 << 30) && a->dw_stride < (1ll << 40), MLA_ERR_UNSUPPORTED,
+            "%s: row stride too large", op);
   // 32-bit byte offsets within a segment (and the stages the ring addresses past it)
   MLA_CHECK((a->M + 8 * kWgSt) * std::max(a->dy_stride, a->x_stride) * 2 < (1ll << 31), MLA_ERR_UNSUPPORTED,
             "%s: operands of 2 GiB or more", op);
