@@ -276,3 +276,25 @@ def test_operator_backward_of_the_attention_sees_the_weights_of_the_forward(tied
                 torch.autograd.grad(y, leaves, dy, create_graph=True)):
         for a, b in zip(got, want):
             assert (a.double() - b.double()).norm() <= 6 * 2.0 ** -9 * b.double().norm()
+
+
+@pytest.mark.parametrize("weights", [torch.bfloat16, torch.float32])
+def test_compiled_training_gradients_equal_eager_ones_to_rounding(weights):
+    """torch.compile keeps torch's layers and the registered operators, in one graph: each gradient within bf16's rounding
+    of the eager branch's."""
+    from contextlib import nullcontext
+    from transformer_amd import MLA, ModelArgs
+    torch.manual_seed(13)
+    with torch.device("cuda"):
+        m = MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=128))  # bf16 RoPE tables
+    m = m.to(weights) if weights == torch.bfloat16 else m
+    x = torch.randn(2, 70, 256, device="cuda").to(weights).requires_grad_(True)
+    dy = torch.randn(2, 70, 256, device="cuda").bfloat16()
+    leaves = [x] + list(m.parameters())
+    amp = nullcontext() if weights == torch.bfloat16 else torch.autocast("cuda", torch.bfloat16)
+    torch._dynamo.reset()
+    with amp:
+        compiled = torch.compile(lambda t: m(t)[0], backend="eager", fullgraph=True)(x)
+        eager = m(x)[0]
+    for a, b in zip(torch.autograd.grad(compiled, leaves, dy), torch.autograd.grad(eager, leaves, dy)):
+        assert a.dtype == b.dtype and (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()

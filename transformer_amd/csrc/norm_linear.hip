@@ -25,8 +25,9 @@
 //     loop has no branch.  With one barrier at the end of a stage every read waited behind it;
 //   * the tile is chosen for the rounds of 256 workgroups (nl_plan in plans.h): M = 24576, N = 2624 made 1056 tiles of
 //     256 x 256, a fifth round of 32 workgroups, where the last 64 columns are now tiles of their own, a quarter as long.
-// Measured calls (the row pass included), before -> now: 24576 x 2624 x 2048 388 -> 337 us, 12288 x 2560 x 1792 137 -> 129,
-// 6555 x 2496 x 1440 109 -> 89, 2735 x 2000 x 1632 63 -> 38, 1000 x 2624 x 2048 68 -> 39, 700 x 512 x 1056 36 -> 19.
+// Measured (kernel trace of 40 calls, medians, the row pass included; one run each on one box), before -> now: 24576 x 2624 x
+// 2048 391 -> 341 us (327 with warm clocks), 12288 x 2560 x 1792 147 -> 134, 6555 x 2496 x 1440 113 -> 92, 2735 x 2000 x 1632
+// 66 -> 41, 1000 x 2624 x 2048 71 -> 40, 700 x 512 x 1056 38 -> 18.  MfmaUtil at the first 33.4 -> 41.0 %.
 #include <cmath>
 
 #include "mla_common.h"

@@ -17,12 +17,14 @@
 // kernel adds the segments' fp32 partials in order (no atomics: the result is bitwise reproducible).  S and the tile
 // come from a cost model (wg_plan in plans.h).
 //
-// Measured (kernel trace, main + segment sum, against the library's product over the same operands):
-//   M = 12288, N x K = 2560 x 1792: 106.5 + 11.8 us (main 1059 TFLOP/s) against 219.6
-//   M = 12288, 1792 x 1792: 74.0 + 12.8 against 112.5;  1792 x 384: 24.2 + 6.8 against 103.6;  896 x 384: 18.2 + 6.2
-//   against 84.6;  M = 3001, 2048 x 2048: 29.8 + 9.6 against 44.0;  2048 x 512: 17.3 + 7.5 against 28.6
-//   M = 8192, 4096 x 2048 (a chunk of the loss): 124.0 + 19.6 against 135.2, a tie, which the loss leaves as it is.
-// A whole training pass of one block (default dims, B = 6, T = 2048) went from 1897 to 1495 us.
+// Measured (kernel trace of 40 calls, medians, main + segment sum with bf16 dW, against the library's product over the same
+// operands in the same run; us):
+//   M = 12288, N x K = 2560 x 1792: 105.2 + 10.8 (main 1072 TFLOP/s) against 218.7;  1792 x 1792: 72.1 + 12.0 against 121.3
+//   1792 x 384: 23.1 + 7.1 against 73.1;  896 x 384: 17.0 + 6.2 against 70.6
+//   M = 3001, 2048 x 2048: 29.7 + 9.3 against 44.5;  2048 x 512: 16.5 + 7.4 against 29.7
+//   M = 8192, 4096 x 2048 (a chunk of the loss): 110.6 + 16.4 against 133.4; M = 3000, 4096 x 1792: 49.2 against 60.1
+// In a training pass of one block (default dims, B = 6, T = 2048) the wide tile runs at 1060 TFLOP/s with MfmaUtil 46.9 %,
+// the narrow one at 671 with 24.3 % (profiles/train_B6_T2048_default.txt); the pass went from 1897 to 1495 us.
 #include <algorithm>
 
 #include "mla_common.h"

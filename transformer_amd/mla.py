@@ -262,9 +262,11 @@ class MLA(nn.Module):
         self.__dict__.pop("_graph_state", None)
 
     def refresh_weights(self):
-        """Forget every weight-derived copy: the bf16 / transposed copies of the few-row products,
-        the concatenated down-projection weight and the recorded decode step.  They are rebuilt
-        from the parameters on next use.  The module notices ordinary parameter updates by their
+        """Forget every weight-derived copy: the bf16 / transposed copies of the few-row products and
+        of the absorbed chunk's W_UK and W_UV, the concatenated down-projection weight and the
+        recorded decode step.  They are rebuilt
+        from the parameters on next use.  (A chunk over per-head K and V reads k_up and v_up
+        themselves, and so do bf16 weights of the few-row products.)  The module notices ordinary parameter updates by their
         storage and version counter; an update that bypasses the version counter (``p.data.copy_``,
         a kernel writing through ``p.data_ptr()``, such as a fused optimizer) must be followed by
         this call before the next inference step."""
