@@ -376,3 +376,33 @@ def test_autocast_does_not_cast_float64_inputs(monkeypatch):
             with pytest.raises(RuntimeError):
                 m._down_all(x)
     assert taken == [torch.bfloat16] * 2
+
+
+@pytest.mark.parametrize("name", ["q_down", "kv_down", "k_up"])
+def test_weights_made_on_each_access_are_not_kept(monkeypatch, name):
+    # a parametrized weight is a fresh tensor: here one at the same address with the same version counter every time, as the
+    # allocator may give it, holding other values
+    from transformer_amd import MLA, ModelArgs
+    import torch.nn as nn
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)  # (asks a GPU)
+    m = MLA(ModelArgs(d_model=256, n_heads=2, d_latent=128, q_lora_rank=128, max_seq_len=64))
+    array = m._modules[name].weight.detach().numpy().copy()
+
+    class Made(nn.Module):
+        weight = property(lambda self: torch.from_numpy(array))
+
+    x = torch.randn(2, 3, 256, generator=torch.Generator().manual_seed(1))
+    with torch.no_grad():
+        with monkeypatch.context() as amp:  # (no GPU: torch turns autocast off)
+            amp.setattr(torch, "is_autocast_enabled", lambda *a: True)
+            amp.setattr(torch, "get_autocast_dtype", lambda *a: torch.bfloat16)
+            assert m._auto_graph_ok(x[:, :1])
+            m._modules[name] = Made()
+            assert not m._auto_graph_ok(x[:, :1])
+        for scale in (1, 2, 4):
+            array *= scale
+            kept = m._cached_weight("down" if name != "k_up" else "k_up:t", lambda: m._modules[name].weight, torch.float64)
+            assert torch.equal(kept, torch.from_numpy(array).double())
+            if name != "k_up":
+                want = torch.cat([m._modules[n].weight for n in ("q_down", "qk_rope", "kv_down")], 0)
+                torch.testing.assert_close(m._down_all(x), x @ want.t())

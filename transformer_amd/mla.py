@@ -146,6 +146,12 @@ def apply_rope(x, cos, sin):
     return y.transpose(1, 2).reshape(*lead, x.size(-2), 64)
 
 
+def _may_be_kept(weights) -> bool:
+    """Whether copies of ``weights`` may be kept by storage and version counter: all are nn.Parameters.  A weight made on
+    each access (a parametrization's, a property's) is a fresh tensor, whose address and version the allocator repeats."""
+    return set(map(type, weights)) == {nn.Parameter}
+
+
 class MLA(nn.Module):
     """DeepSeek-style MLA with decoupled RoPE (transformer.py:128-316) on MI355X kernels."""
 
@@ -193,6 +199,9 @@ class MLA(nn.Module):
         are unchanged (same storage and version counter); autograd off only."""
         params = [self.q_down.weight, self.qk_rope.weight, self.kv_down.weight] if name == "down" else \
             [getattr(self, name.split(":")[0]).weight]
+        if not _may_be_kept(params):
+            with torch.no_grad():
+                return make().to(dtype).contiguous()
         key = tuple((w.data_ptr(), w._version) for w in params) + (dtype,)
         cache = self.__dict__.setdefault("_derived", {})
         hit = cache.get(name)
@@ -213,7 +222,10 @@ class MLA(nn.Module):
         fp32 as the reference's does (transformer.py:215-218, :241-244)."""
         if not AUTO_GRAPH or torch.is_grad_enabled() or not self._plain_projections():
             return False
-        wdt, amp = self._step_weights()[-1].dtype, torch.is_autocast_enabled("cuda")
+        ws = self._step_weights()
+        if not _may_be_kept(ws):
+            return False
+        wdt, amp = ws[-1].dtype, torch.is_autocast_enabled("cuda")
         if amp:
             ok = autocast_bf16() and wdt in (torch.bfloat16, torch.float32) and x.dtype in (torch.bfloat16,
                                                                                             torch.float32)
@@ -347,11 +359,14 @@ class MLA(nn.Module):
                 return training.linear(x.to(dt), *ws, product=_down_product)
             return torch.nn.functional.linear(x, torch.cat(ws, 0))
         dt = torch.get_autocast_dtype("cuda") if amp else ws[0].dtype
-        key = tuple((w.data_ptr(), w._version) for w in ws) + (dt,)
-        if getattr(self, "_down_key", None) != key:
-            self._down_w = torch.cat([w.detach() for w in ws], 0).to(dt)
-            self._down_key = key
-        W = self._down_w
+        if _may_be_kept(ws):
+            key = tuple((w.data_ptr(), w._version) for w in ws) + (dt,)
+            if getattr(self, "_down_key", None) != key:
+                self._down_w = torch.cat([w.detach() for w in ws], 0).to(dt)
+                self._down_key = key
+            W = self._down_w
+        else:
+            W = torch.cat([w.detach() for w in ws], 0).to(dt)
         if not split:
             return training.on_rows(torch.nn.functional.linear, x, W).view(*x.shape[:-1], W.size(0))
         if torch.is_grad_enabled() and x.requires_grad:  # frozen weights, the input's gradient
